@@ -22,7 +22,9 @@
 // rows are staged once in LDS, pair-permuted with per-chunk sums (as the
 // GEMV of qmv.hip stages them); each output row is served by S lanes that
 // stride over its 64-wide groups (32 bytes of W, one s and one b per group
-// and lane), with every W load of a lane issued before the staging.
+// and lane), with every W load of a lane issued before the staging.  With
+// more routes than experts, gather_rows_kernel (below) takes each expert's
+// routes together instead.
 #include <algorithm>
 
 #include "bmx_device.h"
@@ -46,6 +48,7 @@ struct GatherParams {
   int64_t x_rstride, y_rstride;
   int x_bcast, nxb, E, M, N, K;  // nxb: x blocks
   int S;                // lanes per output row (power of two, 1..64)
+  int R;                // routes
 };
 
 template <int MT>
@@ -149,6 +152,287 @@ __global__ void __launch_bounds__(kGThreads) gather_qmv_kernel(const GatherParam
   }
 }
 
+// ---------------------------------------------------------------------------
+// Many routes: every expert's weights read once for all of its rows.
+//
+// gather_qmv_kernel reads a route's whole weight matrix for that route
+// alone, so with R routes over E experts the same weights come from memory
+// (or the caches) R / E times.  Here a workgroup owns one expert and 128
+// output columns.  It finds the expert's routes by scanning the index array
+// (each thread a strip, one prefix sum; no scratch memory, no second
+// launch, so a captured graph replays with new routes), then multiplies
+// their rows in tiles of 16 MT on v_mfma_f32_16x16x32_bf16: A = x rows,
+// read from memory by each lane through its own row pointer; B = the
+// nibbles as bf16 integers 128 + q, lane l holding W row l % 16.  The group
+// decomposition stays as in the per-route kernel, fp32 throughout:
+//   acc = fma(b - 128 s, Sx, fma(s, D, acc)) per group and output,
+// with Sx = x . 1 from one more product against a tile of ones, which puts
+// it in the accumulator's own layout.  Rows past the count repeat the last
+// row and are not stored; a row's result does not depend on its slot.
+//
+// What each operand needs decides where it comes from.  W is read once, so it
+// goes straight to registers: 16 bytes per lane and step of two groups (64
+// contiguous bytes per W row), a chunk of kGChunkK columns ahead.  x is shared
+// by the 8 waves and comes through LDS in chunks, double-buffered, one barrier
+// per chunk; s and b of the workgroup's 256 columns are one contiguous block
+// per array and are staged whole.  (Read per lane and step instead, the 4-byte
+// s and b pieces and the x rows were 85% of the L1 misses, and the kernel ran
+// at the L2's rate: 226 MB of weights in 118 us.)
+constexpr int kGList = 1024;     // routes of the expert listed in LDS at a time
+constexpr int kGChunkK = 256;    // columns of x per LDS chunk
+constexpr int kGXS = kGChunkK + 8;  // LDS row stride of x (odd number of 16-byte units: no bank conflicts)
+constexpr int kGWaves = 8, kGCols = 32 * kGWaves;  // waves and output columns per workgroup
+constexpr int gather_rows_sbstride(int K) { return (K / 128) | 1; }
+constexpr size_t gather_rows_lds(int mt, int K) {
+  return 2ull * 16 * mt * kGXS * 2 + 8ull * kGCols * gather_rows_sbstride(K);
+}
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+
+// the 8 nibbles of a word, in order, as bf16 pairs 128 + q
+__device__ __forceinline__ bf16x8_t nibbles_bf16(uint32_t w, const NibbleK& k) {
+  // pair i: byte i of w under byte i of w >> 4 (one byte permute), then the
+  // low nibbles of both halves over the magic
+  const uint32_t h = w >> 4;
+  uint4 r;
+  r.x = (__builtin_amdgcn_perm(h, w, 0x0c040c00u) & k.mask) | k.magic;
+  r.y = (__builtin_amdgcn_perm(h, w, 0x0c050c01u) & k.mask) | k.magic;
+  r.z = (__builtin_amdgcn_perm(h, w, 0x0c060c02u) & k.mask) | k.magic;
+  r.w = (__builtin_amdgcn_perm(h, w, 0x0c070c03u) & k.mask) | k.magic;
+  return __builtin_bit_cast(bf16x8_t, r);
+}
+
+// MT: 16-row tiles of x
+template <int MT>
+__global__ void __launch_bounds__(64 * kGWaves, MT == 4 ? 2 : 4) gather_rows_kernel(const GatherParams p) {
+  constexpr int T = 64 * kGWaves, NT = 2, D = kGChunkK / 128;
+  constexpr int XU = 16 * MT * (kGChunkK / 8) / T;  // 16-byte units of an x chunk per thread
+  extern __shared__ __align__(16) unsigned char smem[];
+  uint16_t* xs = reinterpret_cast<uint16_t*>(smem);                             // [2][16 MT][kGXS]
+  uint2* sbs = reinterpret_cast<uint2*>(smem + 2 * 16 * MT * kGXS * 2);        // [kGCols][sbstride]: s pair, b pair
+  __shared__ uint16_t list[kGList];
+  __shared__ int wsum[kGWaves];
+  const int K = p.K, S = K / 128, C = K / kGChunkK;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int li = lane & 15, q = lane >> 4;
+  const int e = blockIdx.y, n0 = blockIdx.x * kGCols;
+  // ---- this thread's part of the index array (every T-th): how many
+  // routes are e's, the first 32 of them as a bit mask ----
+  auto mine = [&](int r) {
+    return static_cast<int>(min(p.rhs ? p.rhs[r] : static_cast<uint32_t>(r), static_cast<uint32_t>(p.E - 1))) == e;
+  };
+  int cnt = 0;
+  uint32_t mask = 0;
+  for (int i0 = 0; i0 * T < p.R; i0 += 4) {
+    bool hit[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) hit[u] = mine(min((i0 + u) * T + tid, p.R - 1));
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const bool h = hit[u] && (i0 + u) * T + tid < p.R;
+      cnt += h;
+      if (i0 < 32) mask |= static_cast<uint32_t>(h) << (i0 + u);
+    }
+  }
+  int incl = cnt;
+  for (int off = 1; off < 64; off <<= 1) {
+    const int v = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += v;
+  }
+  if (lane == 63) wsum[wave] = incl;
+  __syncthreads();
+  int total = 0, before = incl - cnt;
+#pragma unroll
+  for (int w = 0; w < kGWaves; w++) {
+    if (w < wave) before += wsum[w];
+    total += wsum[w];
+  }
+  if (total == 0) return;  // uniform
+
+  // ---- this wave's W rows (word offsets inside the expert) ----
+  const uint32_t* we = p.w + static_cast<int64_t>(e) * p.N * (K / 8);
+  uint32_t wo[NT];
+  int n[NT];
+#pragma unroll
+  for (int j = 0; j < NT; j++) {
+    n[j] = n0 + (wave * NT + j) * 16 + li;
+    wo[j] = static_cast<uint32_t>(min(n[j], p.N - 1)) * static_cast<uint32_t>(K / 8) + q * 4;
+  }
+  uint4 wr[D][NT];
+  auto load_w = [&](int u, int step) {
+#pragma unroll
+    for (int j = 0; j < NT; j++) wr[u][j] = *reinterpret_cast<const uint4*>(we + (wo[j] + step * 16));
+  };
+  // ---- s and b of the workgroup's columns (a contiguous block of each) ----
+  const int SB = gather_rows_sbstride(K);
+  {
+    const int64_t base = (static_cast<int64_t>(e) * p.N + n0) * S;  // in words: S = G / 2 per row
+    const uint32_t* se = reinterpret_cast<const uint32_t*>(p.s) + base;
+    const uint32_t* be = reinterpret_cast<const uint32_t*>(p.b) + base;
+    const int words = min(kGCols, p.N - n0) * S;
+    const float rcp = 1.0f / static_cast<float>(S);
+    for (int i0 = 0; i0 < words; i0 += 4 * T) {
+      uint32_t sv[4], bv[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int i = min(i0 + u * T + tid, words - 1);
+        sv[u] = se[i];
+        bv[u] = be[i];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int i = min(i0 + u * T + tid, words - 1);
+        const int row = udiv_small(i, rcp);
+        sbs[row * SB + i - row * S] = make_uint2(sv[u], bv[u]);
+      }
+    }
+  }
+  const NibbleK nk = nibble_consts();
+  const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
+  const f32x4_t zero{0.0f, 0.0f, 0.0f, 0.0f};
+
+  for (int w0 = 0; w0 < total; w0 += kGList) {
+    // ---- routes w0 .. w0 + kGList - 1 of the expert (thread order) ----
+    __syncthreads();  // the last window's list has been read
+    if (cnt > 0) {
+      int idx = before - w0;
+      for (int i = 0; i * T + tid < p.R; i++)
+        if (i < 32 ? (mask >> i) & 1u : static_cast<uint32_t>(mine(i * T + tid))) {
+          if (idx >= 0 && idx < kGList) list[idx] = static_cast<uint16_t>(i * T + tid);
+          idx++;
+        }
+    }
+    __syncthreads();
+    const int rows = min(total - w0, kGList) * p.M;
+    for (int t = blockIdx.z * 16 * MT; t < rows; t += static_cast<int>(gridDim.z) * 16 * MT) {
+      // this thread's part of an x chunk: 16-byte units tid + k T of
+      // [16 MT rows][kGChunkK / 8 units]
+      constexpr int UR = kGChunkK / 8;  // units per row
+      const uint16_t* xp[XU];
+#pragma unroll
+      for (int k = 0; k < XU; k++) {
+        const int unit = tid + k * T;
+        const int j = min(t + unit / UR, rows - 1);
+        const int lr = p.M == 1 ? j : j / p.M, m = j - lr * p.M;
+        const int route = list[lr];
+        const int64_t xb = p.lhs ? min(p.lhs[route], static_cast<uint32_t>(p.nxb - 1)) : route / p.x_bcast;
+        xp[k] = p.x + xb * p.x_rstride + static_cast<int64_t>(m) * K + (unit % UR) * 8;
+      }
+      uint4 xr[XU];
+      auto load_x = [&](int c) {
+#pragma unroll
+        for (int k = 0; k < XU; k++) xr[k] = *reinterpret_cast<const uint4*>(xp[k] + c * kGChunkK);
+      };
+      auto store_x = [&](int c) {
+#pragma unroll
+        for (int k = 0; k < XU; k++) {
+          const int unit = tid + k * T;
+          *reinterpret_cast<uint4*>(xs + ((c & 1) * 16 * MT + unit / UR) * kGXS + (unit % UR) * 8) = xr[k];
+        }
+      };
+      f32x4_t acc[MT][NT];
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] = zero;
+      auto compute = [&](int u, int c) {
+        // lanes q 0, 1 hold a row's 8 words of the step's first group, q 2, 3
+        // of the second; after the swaps every lane holds words
+        // 4 (q & 1) + 2 (q >> 1) + {0, 1} of each
+        uint4 v[NT];
+        uint2 sb[NT];
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+          const auto a = __builtin_amdgcn_permlane32_swap(wr[u][j].x, wr[u][j].z, false, false);
+          const auto b = __builtin_amdgcn_permlane32_swap(wr[u][j].y, wr[u][j].w, false, false);
+          v[j] = make_uint4(a[0], b[0], a[1], b[1]);
+          sb[j] = sbs[((wave * NT + j) * 16 + li) * SB + c * D + u];
+        }
+        const uint16_t* xt = xs + ((c & 1) * 16 * MT + li) * kGXS + u * 128 + (q & 1) * 32 + (q >> 1) * 16;
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+          f32x4_t sx[MT];
+          bf16x8_t xa[MT][2];
+#pragma unroll
+          for (int i = 0; i < MT; i++) {
+            xa[i][0] = *reinterpret_cast<const bf16x8_t*>(xt + i * 16 * kGXS + g * 64);
+            xa[i][1] = *reinterpret_cast<const bf16x8_t*>(xt + i * 16 * kGXS + g * 64 + 8);
+          }
+#pragma unroll
+          for (int i = 0; i < MT; i++) {
+            sx[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][0], ones, zero, 0, 0, 0);
+            sx[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][1], ones, sx[i], 0, 0, 0);
+          }
+#pragma unroll
+          for (int j = 0; j < NT; j++) {
+            const bf16x8_t b0 = nibbles_bf16(g == 0 ? v[j].x : v[j].z, nk);
+            const bf16x8_t b1 = nibbles_bf16(g == 0 ? v[j].y : v[j].w, nk);
+            const float sv = g == 0 ? __uint_as_float(sb[j].x << 16) : __uint_as_float(sb[j].x & 0xffff0000u);
+            const float bv = g == 0 ? __uint_as_float(sb[j].y << 16) : __uint_as_float(sb[j].y & 0xffff0000u);
+            const float bb = __builtin_fmaf(-128.0f, sv, bv);
+            f32x4_t d[MT];
+#pragma unroll
+            for (int i = 0; i < MT; i++) d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][0], b0, zero, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < MT; i++) d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][1], b1, d[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+              for (int r = 0; r < 4; r++)
+                acc[i][j][r] = __builtin_fmaf(bb, sx[i][r], __builtin_fmaf(sv, d[i][r], acc[i][j][r]));
+          }
+        }
+      };
+      // chunk c + 1: x into registers at the top of chunk c, ahead of the W
+      // loads of its steps (loads complete in order, so the x stores at the
+      // bottom leave those in flight), each W step into the registers the
+      // step before it freed.  Loads past the last chunk repeat it.
+      load_x(0);
+#pragma unroll
+      for (int u = 0; u < D; u++) load_w(u, u);
+      store_x(0);
+      __syncthreads();
+      for (int c = 0; c < C; c++) {
+        const int cn = min(c + 1, C - 1);
+        load_x(cn);
+#pragma unroll
+        for (int u = 0; u < D; u++) {
+          __builtin_amdgcn_sched_barrier(0);
+          compute(u, c);
+          __builtin_amdgcn_sched_barrier(0);
+          load_w(u, cn * D + u);
+        }
+        // chunk c - 1's buffer: its reads ended before the last barrier
+        store_x(c + 1);
+        __syncthreads();
+      }
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int j = t + i * 16 + 4 * q + r;
+          if (j >= rows) continue;
+          const int lr = p.M == 1 ? j : j / p.M, m = j - lr * p.M;
+          uint16_t* yr = p.y + static_cast<int64_t>(list[lr]) * p.y_rstride + static_cast<int64_t>(m) * p.N;
+#pragma unroll
+          for (int k = 0; k < NT; k++)
+            if (n[k] < p.N) yr[n[k]] = f2bf(acc[i][k][r]);
+        }
+    }
+  }
+}
+
+template <int MT>
+int launch_gather_rows(const GatherParams& p, int64_t avg, hipStream_t stream) {
+  const size_t lds = gather_rows_lds(MT, p.K);
+  if (int rc = allow_lds(gather_rows_kernel<MT>, lds)) return rc;
+  const dim3 grid((p.N + kGCols - 1) / kGCols, p.E,
+                  static_cast<unsigned>(std::min<int64_t>((avg + 16 * MT - 1) / (16 * MT), 64)));
+  hipLaunchKernelGGL(gather_rows_kernel<MT>, grid, dim3(64 * kGWaves), lds, stream, p);
+  return check_launch("gather_qmm rows");
+}
+
 }  // namespace
 
 int launch_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* s, const uint16_t* b,
@@ -174,7 +458,21 @@ int launch_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* s, c
   const size_t lds = static_cast<size_t>(mt) * (K / 32) * (kGChunk + 4);
   if (lds > 160 * 1024) return set_error(BMX_E_UNSUPPORTED, "gather_qmm: M*K=%d too large", M * K);
   const int rb = 4 * (64 / S);
-  GatherParams p{x, w, s, b, lhs, rhs, y, x_rstride, y_rstride, x_bcast, nxb, E, M, N, K, S};
+  GatherParams p{x, w, s, b, lhs, rhs, y, x_rstride, y_rstride, x_bcast, nxb, E, M, N, K, S, R};
+  // From 1.25 routes per expert on, the expert's weights once for all of its
+  // routes.  128 experts, gate|up 1536 x 2048 and down 2048 x 768, both
+  // calls: 128 routes 54.8 us per route, 54.2 by expert; 192 routes 76.5
+  // against 65; 800 routes 284 against 86; 2664 routes 843 against 160.
+  if (4ll * R >= 5ll * E && E <= 65535 && K % kGChunkK == 0 && aligned(s, 4) && aligned(b, 4) &&
+      gather_rows_lds(4, K) <= 160 * 1024 - 4096 && static_cast<int64_t>(N) * (K / 8) <= UINT32_MAX) {
+    // rows an expert gets on average decide the tile; more tiles than that
+    // are walked by the same workgroup
+    const int64_t rows = static_cast<int64_t>(R) * M;
+    const int64_t avg = (rows + E - 1) / E;
+    return avg <= 8    ? launch_gather_rows<1>(p, avg, stream)
+           : avg <= 48 ? launch_gather_rows<2>(p, avg, stream)
+                       : launch_gather_rows<4>(p, avg, stream);
+  }
   const dim3 grid((N + rb - 1) / rb, R);
   const void* kern = mt == 1   ? reinterpret_cast<const void*>(gather_qmv_kernel<1>)
                      : mt == 2 ? reinterpret_cast<const void*>(gather_qmv_kernel<2>)

@@ -133,3 +133,41 @@ def test_gather_qmm_indexed_errors(gpu):
         with pytest.raises(gpu.BmxError) as ei:
             gpu.gather_qmm_indexed(x, w, s, s, **kw)
         assert ei.value.code == code, kw
+
+
+# From 1.25 routes per expert on, one workgroup multiplies all of an expert's
+# routes (16, 32 or 64 rows a tile, by the average): (E, N, K, M, R, x_bcast,
+# skew); skew sends that share of the routes to expert 1.  Column remainders
+# (N 100, 257), one and several 256-column chunks, rows per route that
+# straddle tiles, an expert above the 1024 routes listed at a time, index
+# arrays beyond the 16384 entries kept as bits, experts without a route.
+ROWS = [(4, 100, 256, 1, 5, 1, 0.0), (16, 257, 768, 1, 40, 8, 0.0), (6, 96, 512, 3, 33, 3, 0.5),
+        (3, 64, 256, 8, 60, 1, 0.9), (5, 288, 512, 1, 200, 4, 0.3), (2, 32, 256, 1, 2500, 1, 0.99),
+        (4, 40, 256, 1, 20011, 1, 0.25), (9, 256, 2048, 1, 300, 1, 0.0)]
+
+
+@pytest.mark.parametrize("E,N,K,M,R,x_bcast,skew", ROWS)
+def test_gather_qmm_by_expert(gpu, orc, E, N, K, M, R, x_bcast, skew):
+    import torch
+
+    print(f"gather_qmm by expert E={E} N={N} K={K} M={M} R={R} x_bcast={x_bcast} skew={skew}", flush=True)
+    (w, s, b), (wq, sq, bq) = _experts(gpu, orc, 5000 + K, E, N, K)
+    rng = np.random.default_rng(R + E)
+    rhs = rng.integers(0, max(E - 1, 1), R).astype(np.uint32)  # the last expert gets no route
+    rhs[rng.random(R) < skew] = 1
+    x = gpu.fill_normal_bf16(5100 + M, (R // x_bcast, M, K))
+    y = gpu.gather_qmm(x, w, s, b, torch.from_numpy(rhs.view(np.int32)).cuda(), x_bcast)
+    # the same routes through lhs_indices, permuted, with ids past the end
+    perm = rng.permutation(R).astype(np.uint32)
+    lhs = (perm // x_bcast).astype(np.uint32)
+    rhs2 = rhs[perm]
+    rhs2[0] = E + 7
+    z = gpu.gather_qmm_indexed(x, w, s, b, torch.from_numpy(lhs.view(np.int32)).cuda(),
+                               torch.from_numpy(rhs2.view(np.int32)).cuda())
+    torch.cuda.synchronize()
+    ref = orc.gather_qmm(torch_bf16_bits(x), wq, sq, bq, rhs, x_bcast)
+    assert _close(torch_bf16_bits(y), ref) > 0.999
+    # a route's bits do not depend on where it stands among its expert's
+    np.testing.assert_array_equal(torch_bf16_bits(z)[1:], torch_bf16_bits(y)[perm[1:]])
+    last = orc.gather_qmm(torch_bf16_bits(x)[lhs[:1]], wq, sq, bq, np.array([E - 1], np.uint32), 1)
+    assert _close(torch_bf16_bits(z)[:1], last) > 0.999
