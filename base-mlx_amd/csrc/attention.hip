@@ -18,7 +18,9 @@
 //   otherwise (prefill): flash attention walking all visible keys,
 //     attn_flash32_kernel (32 queries per wave, a GQA group per workgroup)
 //     where the q heads per kv head are a power of two, else
-//     attn_prefill_kernel (16 queries per wave).
+//     attn_prefill_kernel (16 queries per wave).  Where its query tiles
+//     leave CUs idle, the former splits the keys over the grid and
+//     attn_flash_merge_kernel joins the splits.
 // All run Q K^T and (prefill) P V on the matrix cores.
 #include <math.h>
 
@@ -47,7 +49,7 @@ struct AttnParams {
   int ns;     // key splits
   int causal;
   float scale;
-  int kps;    // keys per split (decode kernel: a multiple of 32, at most 256)
+  int kps;    // keys per split (decode kernel: a multiple of 32, at most 256; flash: whole key blocks, 0 unsplit)
   int local;  // decode kernel: every workgroup of a kv head runs on one XCD (shares its L2)
 };
 
@@ -1046,6 +1048,13 @@ __global__ void __launch_bounds__(64 * NW) attn_prefill_kernel(const AttnParams 
 //     l as well, and its rescale by exp(m_old - m_new) needs no shuffle.
 // Half the LDS operand reads per product of the 16-query layout, and the
 // cross-lane reductions of a block halve.
+//
+// Key split (p.kps > 0): one workgroup fills a CU (133 KB of LDS), so a
+// chunk of 203 tokens over 8 kv heads is 32 of them on 256 CUs, each walking
+// every key.  With the keys over blockIdx.z each workgroup walks p.kps of
+// them and leaves (O, m, l) in fp32 for attn_flash_merge_kernel: 32 q heads,
+// 203 tokens over 3000 cached 133 -> 51 us, 64 over 4096 165 -> 40, 513 over
+// none unchanged (flash_split_blocks decides).
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 // Its LDS rows (strides chosen with a bank-conflict probe of each access:
 // 16-byte operand reads of 32 consecutive rows are conflict-free at 272
@@ -1077,7 +1086,13 @@ __global__ void __launch_bounds__(512) attn_flash32_kernel(const AttnParams p) {
   const int offset = p.offset_dev ? *p.offset_dev : p.offset;
   const int L = offset + p.M;
   const int kend = p.causal ? min(L, offset + min(t0 + TQ, p.M)) : L;
-  const int nkb = (kend + kFaK - 1) / kFaK;
+  // key blocks of this workgroup: all the tile sees, or (split) the
+  // blockIdx.z-th p.kps keys of them
+  const int nkb_all = (kend + kFaK - 1) / kFaK;
+  const int bps = p.kps / kFaK;
+  const int jb0 = bps ? static_cast<int>(blockIdx.z) * bps : 0;
+  if (jb0 >= nkb_all) return;  // uniform
+  const int nkb = bps ? min(jb0 + bps, nkb_all) : nkb_all;
   const int tw = t0 + 32 * (wave / HG);  // the wave's first query
   const int t = tw + j;                  // this lane's query
   const int64_t hbase = static_cast<int64_t>(kvh) * p.cap * kD;
@@ -1183,15 +1198,16 @@ __global__ void __launch_bounds__(512) attn_flash32_kernel(const AttnParams p) {
 
   // two register sets: block jb + 2 is requested while block jb's products
   // run and block jb + 1 moves from registers into LDS
-  Stage sg0 = load_block(0);
-  Stage sg1 = load_block(min(1, nkb - 1) * kFaK);
+  Stage sg0 = load_block(jb0 * kFaK);
+  Stage sg1 = load_block(min(jb0 + 1, nkb - 1) * kFaK);
   for (int i = threadIdx.x; i < kFaSatWords; i += 512) vsat[i] = 0u;
   __syncthreads();
-  store_block(sg0, 0, 0);
+  store_block(sg0, 0, jb0);
   __syncthreads();
   auto iter = [&](const int jb, auto par_c) {
     constexpr int P = decltype(par_c)::value;
-    const int buf = jb & 1, k0 = jb * kFaK;
+    constexpr int buf = P;
+    const int k0 = jb * kFaK;
     const bool more = jb + 1 < nkb;
     if constexpr (P == 0) sg0 = load_block(min(jb + 2, nkb - 1) * kFaK);
     else sg1 = load_block(min(jb + 2, nkb - 1) * kFaK);
@@ -1315,9 +1331,24 @@ __global__ void __launch_bounds__(512) attn_flash32_kernel(const AttnParams p) {
     if (more) store_block(P == 0 ? sg1 : sg0, buf ^ 1, jb + 1);
     __syncthreads();
   };
-  for (int jb = 0; jb < nkb; jb += 2) {
+  for (int jb = jb0; jb < nkb; jb += 2) {
     iter(jb, std::integral_constant<int, 0>{});
     if (jb + 1 < nkb) iter(jb + 1, std::integral_constant<int, 1>{});
+  }
+  if (bps && nkb_all > bps) {
+    // ---- one of several splits of this tile: unnormalised partials ----
+    if (t < p.M) {
+      const int64_t row = (static_cast<int64_t>(blockIdx.z) * p.Hq + h) * p.M + t;
+      if (hf == 0) *reinterpret_cast<float2*>(p.part_ml + row * 2) = make_float2(m_run, l_run);
+      float* orow = p.part_o + row * kD + 4 * hf;
+#pragma unroll
+      for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++)
+          *reinterpret_cast<float4*>(orow + 32 * dt + 8 * r4) =
+              make_float4(o[dt][4 * r4], o[dt][4 * r4 + 1], o[dt][4 * r4 + 2], o[dt][4 * r4 + 3]);
+    }
+    return;
   }
   // ---- normalise and write: dims 32 dt + 8 r4 + 4 hf .. + 3 of query t ----
   if (t < p.M) {
@@ -1335,6 +1366,51 @@ __global__ void __launch_bounds__(512) attn_flash32_kernel(const AttnParams p) {
         *reinterpret_cast<uint2*>(orow + 32 * dt + 8 * r4) = make_uint2(w0, w1);
       }
   }
+}
+
+// Merges the splits of attn_flash32_kernel: 32 lanes per (head, query) row,
+// 4 dims per lane.  A row's tile of tq tokens has ceil(visible keys / kps)
+// splits; rows of unsplit tiles were written by the attention kernel.
+__global__ void __launch_bounds__(256) attn_flash_merge_kernel(const AttnParams p) {
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * 8 + (threadIdx.x >> 5);
+  const int64_t rows = static_cast<int64_t>(p.Hq) * p.M;
+  if (row >= rows) return;
+  const int h = static_cast<int>(row / p.M), t = static_cast<int>(row - static_cast<int64_t>(h) * p.M);
+  const int offset = p.offset_dev ? *p.offset_dev : p.offset;
+  const int L = offset + p.M;
+  const int kend = p.causal ? min(L, offset + min(t / p.tq * p.tq + p.tq, p.M)) : L;
+  const int ns = (kend + p.kps - 1) / p.kps;
+  if (ns < 2) return;
+  const int d = (threadIdx.x & 31) * 4;
+  constexpr int B = 4;  // splits in flight
+  float m = -INFINITY, l = 0.0f;
+  float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int z0 = 0; z0 < ns; z0 += B) {
+    float2 ml[B];
+    float4 v[B];
+#pragma unroll
+    for (int u = 0; u < B; u++) {
+      const int64_t r = static_cast<int64_t>(min(z0 + u, ns - 1)) * rows + row;
+      ml[u] = *reinterpret_cast<const float2*>(p.part_ml + r * 2);
+      v[u] = *reinterpret_cast<const float4*>(p.part_o + r * kD + d);
+    }
+#pragma unroll
+    for (int u = 0; u < B; u++) {
+      if (z0 + u >= ns || ml[u].x == -INFINITY) continue;  // no key of the split visible to the row
+      const float mn = fmaxf(m, ml[u].x);
+      const float wa = __builtin_amdgcn_exp2f(m - mn), wb = __builtin_amdgcn_exp2f(ml[u].x - mn);
+      l = l * wa + ml[u].y * wb;
+      a.x = a.x * wa + v[u].x * wb;
+      a.y = a.y * wa + v[u].y * wb;
+      a.z = a.z * wa + v[u].z * wb;
+      a.w = a.w * wa + v[u].w * wb;
+      m = mn;
+    }
+  }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  *reinterpret_cast<uint2*>(p.out + static_cast<int64_t>(t) * p.Hq * kD + h * kD + d) =
+      make_uint2(static_cast<uint32_t>(f2bf(a.x * inv)) | (static_cast<uint32_t>(f2bf(a.y * inv)) << 16),
+                 static_cast<uint32_t>(f2bf(a.z * inv)) | (static_cast<uint32_t>(f2bf(a.w * inv)) << 16));
 }
 
 }  // namespace
@@ -1469,6 +1545,50 @@ int check_attention_shape(int Hq, int Hkv, int M, int D, int cap, int offset, co
   return BMX_OK;
 }
 
+// Key blocks per split of a flash attention over `groups` head groups and
+// the key-block counts of its query tiles (a function of `tiles`, tq and the
+// mask): one workgroup per CU, so the time is about that of the longest
+// workgroup or of the mean load, in units of one key block (2.4 us measured),
+// with 2 blocks' worth per workgroup for its start and end and, once split,
+// 2 for the merge launch and the partials' traffic (Hq M 520 bytes per split,
+// written and read back at about 4 TB/s).  0: not split.
+int flash_split_blocks(int groups, int tiles, int tq, int Hq, int M, int offset, bool causal, size_t part_floats,
+                       int64_t* splits_out) {
+  constexpr int kCus = 256;
+  auto blocks = [&](int i) {
+    const int kend = causal ? offset + std::min((i + 1) * tq, M) : offset + M;
+    return (kend + kFaK - 1) / kFaK;
+  };
+  const int most = blocks(tiles - 1);
+  *splits_out = 1;
+  if (tiles > 2 * kCus || most < 4) return 0;
+  auto cost = [&](int bps) {
+    int64_t wgs = 0, sum = 0;
+    for (int i = 0; i < tiles; i++) {
+      const int n = blocks(i);
+      wgs += (n + bps - 1) / bps;
+      sum += n;
+    }
+    const double mean = static_cast<double>(groups) * (sum + 2 * wgs) / kCus;
+    const double ns = (most + bps - 1) / bps;
+    const double merge = ns > 1 ? 2.0 + ns * Hq * M * 1040.0 / 4.0e6 / 2.4 : 0.0;
+    return std::max(mean, bps + 2.0) * (groups * wgs > kCus ? 1.1 : 1.0) + merge;
+  };
+  int best = 0;
+  double least = cost(most) * 0.9;  // a split has to promise 10%
+  for (int ns = 2; ns <= 64 && (most + ns - 1) / ns >= 2; ns++) {
+    const int bps = (most + ns - 1) / ns, n = (most + bps - 1) / bps;
+    if (static_cast<size_t>(n) * Hq * M * (kD + 2) > part_floats) break;
+    const double c = cost(bps);
+    if (c < least) {
+      least = c;
+      best = bps;
+      *splits_out = n;
+    }
+  }
+  return best;
+}
+
 }  // namespace
 
 void attention_prepare(hipStream_t stream) { (void)xcd_local_ok(stream); }
@@ -1495,8 +1615,23 @@ int launch_attention(const uint16_t* q, const uint16_t* k, const uint16_t* v, ui
     if (int e = allow_lds_ptr(reinterpret_cast<const void*>(kern), kF32Lds)) return e;
     const int tq = 256 / hg, tiles = (M + tq - 1) / tq;
     if (tiles > 65535) return set_error(BMX_E_SHAPE, "attention: M=%d too large for one prefill launch", M);
-    hipLaunchKernelGGL(kern, dim3(Hkv * (rep / hg), tiles), dim3(512), kF32Lds, stream, p);
-    return check_launch("attention_prefill");
+    // few or uneven query tiles: the keys split over the grid's z axis where
+    // the workspace holds the partials (positions known on the host, so the
+    // grid has every split)
+    int64_t ns = 1;
+    if (ws && aligned(ws, 16) && ws_floats > kCounters && !offset_dev) {
+      const int groups = Hkv * (rep / hg);
+      p.kps = kFaK * flash_split_blocks(groups, tiles, tq, Hq, M, offset, p.causal != 0, ws_floats - kCounters, &ns);
+      p.part_o = ws + kCounters;
+      p.part_ml = p.part_o + static_cast<size_t>(ns) * Hq * M * kD;
+      p.tq = tq;
+    }
+    hipLaunchKernelGGL(kern, dim3(Hkv * (rep / hg), tiles, static_cast<unsigned>(ns)), dim3(512), kF32Lds, stream, p);
+    if (int e = check_launch("attention_prefill")) return e;
+    if (ns == 1) return BMX_OK;
+    hipLaunchKernelGGL(attn_flash_merge_kernel, dim3(static_cast<unsigned>((static_cast<int64_t>(Hq) * M + 7) / 8)),
+                       dim3(256), 0, stream, p);
+    return check_launch("attention_merge");
   };
   if (rep % 8 == 0) return launch32(attn_flash32_kernel<8>, 8);
   if (rep == 4) return launch32(attn_flash32_kernel<4>, 4);

@@ -219,9 +219,10 @@ int bmx_qk_norm_rope_kv(const bmx_bf16 *q, const bmx_bf16 *k, const bmx_bf16 *v,
  * kv head h / (n_heads / n_kv_heads); for M > 1 query t sees keys
  * j <= offset + t.  `workspace` (may be NULL: no key split) holds arrival
  * counters and split partials; bmx_attention_workspace_bytes(n_heads, M) is
- * enough, 16-byte aligned.  It must be zero-filled before its first use; every call leaves
- * the counters zero again, so it is reused as is.  Calls that share one
- * workspace must not run concurrently.
+ * enough, 16-byte aligned (a call of many tokens splits its keys only where
+ * the workspace it is given has room).  It must be zero-filled before its
+ * first use; every call leaves the counters zero again, so it is reused as
+ * is.  Calls that share one workspace must not run concurrently.
  * Replaces: mlx_rs::fast::scaled_dot_product_attention with the
  *   causal_mask_offset mask (crates/base-mlx-core/src/model/qwen3.rs:491-518,
  *   629-653). */

@@ -117,6 +117,35 @@ def test_attention_prefill_v_beyond_fp16_range(gpu, orc, M, offset):
     assert _close(yb, ref, ulps=2, floor=2e-3) > 0.999
 
 
+# (Hq, Hkv, M, offset): few query tiles over many keys, where the flash kernel
+# splits the keys given a workspace: 4, 2, 8 and 1 q heads per kv head, a last
+# tile of 1 token, key counts around a block, splits whose keys the first
+# rows of a tile do not see
+@pytest.mark.parametrize("Hq,Hkv,M,offset", [(32, 8, 70, 3000), (16, 8, 129, 700), (64, 8, 17, 943), (8, 8, 257, 1000),
+                                             (32, 8, 513, 1111), (32, 8, 65, 448)])
+def test_attention_flash_key_split(gpu, orc, Hq, Hkv, M, offset):
+    import torch
+
+    cap = offset + M + 5
+    q = gpu.fill_normal_bf16(61, (Hq, M, 128))
+    kc = gpu.fill_normal_bf16(62, (Hkv, cap, 128))
+    vc = gpu.fill_normal_bf16(63, (Hkv, cap, 128))
+    vc[:, offset - 64:offset] *= 2.0 ** 17  # one block or two beyond fp16's range
+    scale = 1 / np.sqrt(128)
+    ref = orc.sdpa(torch_bf16_bits(q), torch_bf16_bits(kc), torch_bf16_bits(vc), offset + M, offset, True,
+                   np.float32(scale))
+    ws = gpu.attention_workspace(Hq, 16)
+    one = torch_bf16_bits(gpu.attention(q, kc, vc, offset, scale, use_workspace=False))
+    for _ in range(2):  # the workspace reused as it was left
+        yb = torch_bf16_bits(gpu.attention(q, kc, vc, offset, scale, workspace=ws))
+        assert max_rel_err(bf16_to_f32(yb), bf16_to_f32(ref)) < 1e-2
+        assert _close(yb, ref, ulps=2, floor=2e-3) > 0.999
+    assert not ws[:8192].any()  # the decode kernel's counters untouched
+    # a workspace with no room for two splits: the unsplit kernel's bits
+    small = torch.zeros(8192 + 100, dtype=torch.float32, device="cuda")
+    np.testing.assert_array_equal(torch_bf16_bits(gpu.attention(q, kc, vc, offset, scale, workspace=small)), one)
+
+
 def test_attention_workspace_reuse(gpu, orc):
     """One zero-filled workspace over calls of different split counts and row
     tilings: the arrival counters come back to zero after every call."""
