@@ -95,7 +95,7 @@ int launch_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* s, const ui
 // The same x times up to 3 weights (q, k, v of a layer) with separate
 // outputs y[i] of n[i] columns: one launch when every n[i] is a multiple of
 // 128 and K does not split, else one launch_qmm per weight.  Each output is
-// bit-identical to its own launch_qmm without a K split.
+// its own launch_qmm's up to the order of the fp32 sums.
 int launch_qmm_segments(const uint16_t* x, int nseg, const uint32_t* const* w, const uint16_t* const* s,
                         const uint16_t* const* b, uint16_t* const* y, const int* n, int M, int K, float* ws,
                         size_t ws_floats, hipStream_t stream);
@@ -107,10 +107,13 @@ enum QmmEpilogue { QMM_STORE = 0, QMM_RESIDUAL = 1, QMM_SWIGLU = 2, QMM_QKV_ROPE
 int launch_qmm_epi(QmmEpilogue epi, const uint16_t* x, const uint32_t* w, const uint16_t* s, const uint16_t* b,
                    const uint32_t* w2, const uint16_t* s2, const uint16_t* b2, const uint16_t* res, uint16_t* y, int M,
                    int N, int K, float* ws, size_t ws_floats, hipStream_t stream);
+// Whether launch_qmm_epi (one_launch: launch_qmm_segments, N the sum) takes
+// the few-rows kernel for the product, which reads MLX-layout weights.
+bool qmm_few_rows(QmmEpilogue epi, int M, int N, int K, bool one_launch);
 // The same products over group-major copies of the weights (launch_qmm_repack):
 // W as [K/64][N][8] words and s|b as [K/64][N] words s | b << 16, so the
 // rows of one group in a tile are contiguous.  Bit-identical to the MLX-layout
-// launches; kNoFit (nothing launched) where the one-launch segments form or
+// launches of the tile kernel; kNoFit (nothing launched) where the one-launch segments form or
 // the SwiGLU form does not fit, for the caller's MLX-layout fallback.
 int launch_qmm_epi_gm(QmmEpilogue epi, const uint16_t* x, const uint32_t* w, const uint32_t* sb, const uint32_t* w2,
                       const uint32_t* sb2, const uint16_t* res, uint16_t* y, int M, int N, int K, float* ws,

@@ -21,7 +21,7 @@
 // straight from memory into one of two LDS tiles (global_load_lds_dwordx4)
 // a group ahead, W through registers.  When the tile grid is small, K is
 // split over workgroups: fp32 partial tiles go to a workspace and a
-// reduction kernel writes y.
+// reduction kernel writes y.  Few rows of x take qmm_slab.hip instead.
 //
 // Epilogues (the prefill's MLX op sequence fused, with the same bf16
 // roundings): store; residual, y = res + bf16(x W^T) (qwen3.rs:520-521, 541);
@@ -34,15 +34,10 @@
 #include <map>
 #include <mutex>
 
-#include "bmx_device.h"
+#include "qmm_device.h"
 
 namespace bmx {
 namespace {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-typedef __attribute__((ext_vector_type(2))) float f32x2_t;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
 
 constexpr int QBM = 128, QBN = 128, QT = 256;  // tile rows of x, of W; threads
 // LDS tiles: 64 bf16 (128 bytes, 8 chunks of 16 bytes) per row, unpadded;
@@ -78,47 +73,6 @@ bool qmm_tile160(int M, int N) {
   return t160 > 384 && t160 <= 512 && (t128 + 255) / 256 * 128 > (t160 + 255) / 256 * 160;
 }
 __device__ __forceinline__ int swz(int row, int chunk) { return row * RS + ((chunk ^ (row & 7)) << 3); }
-
-struct QmmParams {
-  const uint16_t* x;   // [M, K]
-  const uint32_t* w;   // [N, K/8] (SwiGLU: gate)
-  const uint16_t* s;   // [N, K/64]
-  const uint16_t* b;   // [N, K/64]
-  const uint32_t* w2;  // SwiGLU: up weight, scales and biases
-  const uint16_t* s2;
-  const uint16_t* b2;
-  const uint16_t* res;  // residual: [M, N] (may alias y)
-  uint16_t* y;          // [M, N] bf16 (one split)
-  float* part;          // [splits, M, N] fp32 partials (several splits)
-  int M, N, K;
-  int gps;     // groups per split
-  int mtiles;  // row tiles of x (the grid's x dimension enumerates mtiles x column tiles)
-  int xcd;     // tile order: 0 row-major; XCD-grouped 1 column-major, 2 row-major
-  // Store epilogue over up to 3 column segments (q | k | v of one layer in
-  // one launch): segment i covers output columns [seg_n0[i], seg_n0[i+1])
-  // of the launch (multiples of the tile width) with its own W, s, b and y
-  // (y row stride = the segment's width).  nseg = 0: the plain product.
-  int nseg;
-  int seg_n0[4];
-  const uint32_t* seg_w[3];
-  const uint16_t* seg_s[3];
-  const uint16_t* seg_b[3];
-  uint16_t* seg_y[3];
-  // Group-major weights (the model's prefill copy): w, w2 and seg_w hold
-  // [K/64][N][8] words (each row's 64 nibbles of one group, rows of a group
-  // consecutive), and sb, sb2 and seg_sb [K/64][N] words s | b << 16, so a
-  // tile's W and s|b of one group are contiguous
-  const uint32_t* sb;
-  const uint32_t* sb2;
-  const uint32_t* seg_sb[3];
-  // QMM_QKV_ROPE: where the normed / rotated rows go
-  QkvRopeOut rope;
-};
-
-// two floats -> packed bf16 pair, round to nearest even (v_cvt_pk_bf16_f32)
-__device__ __forceinline__ uint32_t pk_bf16(float lo, float hi) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo, hi}), bf16x2_t));
-}
 
 // BN: W rows per tile, 128 (waves of 64 x 64) or 256 (waves of 64 x 128:
 // the x tile serves twice the W rows, for large grids).  GM: weights in the
@@ -279,20 +233,7 @@ __global__ void __launch_bounds__(2 * QM, QM == QBM ? 2 : 1) qmm_kernel(const Qm
     // sv, bv: the row's scale and bias as floats
     auto put_row = [&](int row, const uint4 wq, float sv, float bv) {
       auto put_word = [&](int chunk, uint32_t word) {
-        // nibble k of the word is value k: even k in the low nibble of byte
-        // k/2, odd k in the high nibble
-        uint32_t lo = word & 0x0f0f0f0fu, hi = (word >> 4) & 0x0f0f0f0fu;
-        // opaque, so each byte converts with one v_cvt_f32_ubyte<n> instead of
-        // a bit-field extract and a convert
-        asm volatile("" : "+v"(lo), "+v"(hi));
-        uint4 o;
-        o.x = pk_bf16(fmaf(sv, static_cast<float>(lo & 0xffu), bv), fmaf(sv, static_cast<float>(hi & 0xffu), bv));
-        o.y = pk_bf16(fmaf(sv, static_cast<float>((lo >> 8) & 0xffu), bv),
-                      fmaf(sv, static_cast<float>((hi >> 8) & 0xffu), bv));
-        o.z = pk_bf16(fmaf(sv, static_cast<float>((lo >> 16) & 0xffu), bv),
-                      fmaf(sv, static_cast<float>((hi >> 16) & 0xffu), bv));
-        o.w = pk_bf16(fmaf(sv, static_cast<float>(lo >> 24), bv), fmaf(sv, static_cast<float>(hi >> 24), bv));
-        *reinterpret_cast<uint4*>(wt + swz(row, chunk)) = o;
+        *reinterpret_cast<uint4*>(wt + swz(row, chunk)) = qmm_dequant_word(word, sv, bv);
       };
       put_word(wh * 4, wq.x);
       put_word(wh * 4 + 1, wq.y);
@@ -650,6 +591,9 @@ const void* qmm_kernel_rows(bool gm, int qm) {
   return qm > QBM ? qmm_kernel_for<EPI, BN, 2 * QBM>(gm) : qmm_kernel_for<EPI, BN>(gm);
 }
 
+// (MLX-layout weights, s and b 4-byte aligned)
+bool slab_aligned(const void* s, const void* b) { return aligned(s, 4) && aligned(b, 4); }
+
 // The GEMM with an epilogue over MLX-layout (sb == nullptr) or group-major
 // weights (w, w2 and sb, sb2 in the layout of QmmParams)
 int qmm_epi_impl(QmmEpilogue epi, const uint16_t* x, const uint32_t* w, const uint16_t* s, const uint16_t* b,
@@ -671,8 +615,12 @@ int qmm_epi_impl(QmmEpilogue epi, const uint16_t* x, const uint32_t* w, const ui
   const int cols = epi == QMM_SWIGLU ? bn / 2 : bn;
   int splits = 1, gps = K / 64;
   if (bn == 128) qmm_split(M, N, K, &splits, &gps, cols);
+  // few rows: the slab kernel, with no more K splits (so no more partials)
+  // than the tile kernel takes
+  const bool slab_ok = !gm && slab_aligned(s, b) && (epi != QMM_SWIGLU || slab_aligned(s2, b2));
+  const SlabPlan slab = slab_ok ? slab_plan(epi, M, N, K, splits) : SlabPlan{};
   // SwiGLU needs both products of an output in one workgroup: no K split
-  if (epi == QMM_SWIGLU && splits > 1) return kNoFit;
+  if (epi == QMM_SWIGLU && splits > 1 && !slab.fits) return kNoFit;
   // 256-row x tiles on 8 waves (one workgroup per CU) from M = 2048 on:
   // for 160- and 256-column tiles, and for 128-column tiles where their grid
   // fills its last round of 256 CUs to 90% or more.  Public entry point,
@@ -696,7 +644,7 @@ int qmm_epi_impl(QmmEpilogue epi, const uint16_t* x, const uint32_t* w, const ui
   QmmParams p{x, w, s, b, w2, s2, b2, res, y, nullptr, M, N, K, gps, mtiles, xcd};
   p.sb = sb;
   p.sb2 = sb2;
-  if (splits > 1) {
+  if (splits > 1 && epi != QMM_SWIGLU) {
     if (int rc = split_scratch(static_cast<size_t>(splits) * M * N, ws, ws_floats, stream, &p.part)) return rc;
   }
   const dim3 grid(static_cast<unsigned>(mtiles) * ntiles, 1, splits);
@@ -715,8 +663,9 @@ int qmm_epi_impl(QmmEpilogue epi, const uint16_t* x, const uint32_t* w, const ui
                                  : (epi == QMM_SWIGLU     ? qmm_kernel_rows<QMM_SWIGLU, 128>(gm, qm)
                                     : epi == QMM_RESIDUAL ? qmm_kernel_rows<QMM_RESIDUAL, 128>(gm, qm)
                                                           : qmm_kernel_rows<QMM_STORE, 128>(gm, qm));
-  const int rc = launch(kern, bn);
+  const int rc = slab.fits ? launch_qmm_slab(epi, p, slab, stream) : launch(kern, bn);
   if (rc) return rc;
+  if (slab.fits) splits = slab.splits;
   if (splits > 1) {
     const int64_t mn = static_cast<int64_t>(M) * N;
     const uint16_t* r = epi == QMM_RESIDUAL ? res : nullptr;
@@ -752,9 +701,17 @@ int qmm_segments_impl(const uint16_t* x, int nseg, const uint32_t* const* w, con
   } else if (one) {
     qmm_split(M, ntot, K, &splits, &gps, QBN);
   }
+  // few rows: one launch of the slab kernel, K unsplit (128-column segments
+  // are whole tiles of either width)
+  SlabPlan slab{};
+  if (one && !gm && nseg > 1) {
+    bool ok = true;
+    for (int i = 0; i < nseg; i++) ok = ok && slab_aligned(s[i], b[i]);
+    if (ok) slab = slab_plan(QMM_STORE, M, ntot, K, 1);
+  }
   // one launch when every segment is whole tiles and K is not split (the
   // reduction writes one y); else a launch per segment
-  if (!one || splits > 1 || (M + QBM - 1) / QBM > 65535) {
+  if (!slab.fits && (!one || splits > 1 || (M + QBM - 1) / QBM > 65535)) {
     if (gm) return kNoFit;
     for (int i = 0; i < nseg; i++)
       if (int rc = launch_qmm(x, w[i], s[i], b[i], y[i], M, n[i], K, ws, ws_floats, stream)) return rc;
@@ -775,6 +732,7 @@ int qmm_segments_impl(const uint16_t* x, int nseg, const uint32_t* const* w, con
     c += n[i];
   }
   for (int i = nseg; i < 4; i++) p.seg_n0[i] = c;
+  if (slab.fits) return launch_qmm_slab(QMM_STORE, p, slab, stream);
   const void* kern = wide ? qmm_kernel_for<QMM_STORE, 256>(gm) : qmm_kernel_for<QMM_STORE, 128>(gm);
   if (int rc = allow_lds_ptr(kern, qmm_lds(bn))) return rc;
   void* args[] = {&p};
@@ -786,6 +744,13 @@ int qmm_segments_impl(const uint16_t* x, int nseg, const uint32_t* const* w, con
 }
 
 }  // namespace
+
+bool qmm_few_rows(QmmEpilogue epi, int M, int N, int K, bool one_launch) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 64) return false;
+  int splits, gps;
+  qmm_split(M, N, K, &splits, &gps, epi == QMM_SWIGLU ? QBN / 2 : QBN);
+  return slab_plan(epi, M, N, K, one_launch ? 1 : splits).fits;
+}
 
 int launch_qmm_epi(QmmEpilogue epi, const uint16_t* x, const uint32_t* w, const uint16_t* s, const uint16_t* b,
                    const uint32_t* w2, const uint16_t* s2, const uint16_t* b2, const uint16_t* res, uint16_t* y, int M,

@@ -205,6 +205,16 @@ int qmv(const bmx_qwen3* m, const uint16_t* x, int M, const QLin& w, uint16_t* y
   return launch_qmv(p, QMV_STORE, st);
 }
 
+// m->x += x w^T (prefill): the group-major copy, or MLX's layout where the
+// few-rows kernel takes the product
+int qmm_residual(const bmx_qwen3* m, const uint16_t* x, const QLin& w, int M, hipStream_t st) {
+  if (qmm_few_rows(QMM_RESIDUAL, M, w.N, w.K, false))
+    return launch_qmm_epi(QMM_RESIDUAL, x, w.w, w.s, w.b, nullptr, nullptr, nullptr, m->x, m->x, M, w.N, w.K, m->qmm_ws,
+                          m->qmm_ws_floats, st);
+  return launch_qmm_epi_gm(QMM_RESIDUAL, x, w.wt, w.sbt, nullptr, nullptr, m->x, m->x, M, w.N, w.K, m->qmm_ws,
+                           m->qmm_ws_floats, st);
+}
+
 const QLin& head_of(const bmx_qwen3* m) { return m->cfg.tied ? m->embed : m->lm_head; }
 
 // One forward over M tokens whose ids are already in m->ids, at position
@@ -259,12 +269,14 @@ int forward_device(bmx_qwen3* m, bmx_kv_cache* c, int M, int offset, const int* 
       uint16_t* y3[3] = {m->q, m->k, m->v};
       const int n3[3] = {qd, kvd, kvd};
       int rc = kNoFit;
-      if (rope_gemm) {
+      const bool few = qmm_few_rows(QMM_STORE, M, qd + 2 * kvd, H, true);
+      if (rope_gemm && !few) {
         const QkvRopeOut ro{L.q_norm, L.k_norm, m->qr, c->k(l), c->v(l), m->rope_cs, pos_dev, offset, c->cap, cf.eps};
         rc = launch_qmm_qkv_rope_gm(m->h, wt3, sb3, n3, M, H, ro, st);
         if (rc == BMX_OK) roped = true;
       }
-      if (rc == kNoFit) rc = launch_qmm_segments_gm(m->h, 3, wt3, sb3, y3, n3, M, H, m->qmm_ws, m->qmm_ws_floats, st);
+      if (rc == kNoFit && !few)
+        rc = launch_qmm_segments_gm(m->h, 3, wt3, sb3, y3, n3, M, H, m->qmm_ws, m->qmm_ws_floats, st);
       if (rc == kNoFit) {
         const uint32_t* w3[3] = {L.p[SLOT_Q].w, L.p[SLOT_K].w, L.p[SLOT_V].w};
         const uint16_t* s3[3] = {L.p[SLOT_Q].s, L.p[SLOT_K].s, L.p[SLOT_V].s};
@@ -307,9 +319,7 @@ int forward_device(bmx_qwen3* m, bmx_kv_cache* c, int M, int offset, const int* 
       p.part_floats = m->qmm_ws_floats;
       if (int rc = launch_qmv(p, QMV_RESIDUAL, st)) return rc;
     } else {
-      if (int rc = launch_qmm_epi_gm(QMM_RESIDUAL, m->att, L.p[SLOT_O].wt, L.p[SLOT_O].sbt, nullptr, nullptr, m->x,
-                                     m->x, M, H, qd, m->qmm_ws, m->qmm_ws_floats, st))
-        return rc;
+      if (int rc = qmm_residual(m, m->att, L.p[SLOT_O], M, st)) return rc;
     }
     // ---- mlp_block + residual (kernels.rs:55-78; qwen3.rs:523-541) ----
     if (M <= 8) {
@@ -341,8 +351,12 @@ int forward_device(bmx_qwen3* m, bmx_kv_cache* c, int M, int offset, const int* 
       if (int rc = launch_rms_norm(m->x, L.post_norm, m->h, M, H, cf.eps, st)) return rc;
       // gate, up and SwiGLU in one GEMM when it does not split K, else three steps
       const QLin &gw = L.p[SLOT_GATE], &uw = L.p[SLOT_UP];
-      const int fused = launch_qmm_epi_gm(QMM_SWIGLU, m->h, gw.wt, gw.sbt, uw.wt, uw.sbt, nullptr, m->a, M, I, H,
-                                          m->qmm_ws, m->qmm_ws_floats, st);
+      const int fused =
+          qmm_few_rows(QMM_SWIGLU, M, I, H, true)
+              ? launch_qmm_epi(QMM_SWIGLU, m->h, gw.w, gw.s, gw.b, uw.w, uw.s, uw.b, nullptr, m->a, M, I, H, m->qmm_ws,
+                               m->qmm_ws_floats, st)
+              : launch_qmm_epi_gm(QMM_SWIGLU, m->h, gw.wt, gw.sbt, uw.wt, uw.sbt, nullptr, m->a, M, I, H, m->qmm_ws,
+                                  m->qmm_ws_floats, st);
       if (fused != kNoFit) {
         if (fused) return fused;
       } else {
@@ -350,9 +364,7 @@ int forward_device(bmx_qwen3* m, bmx_kv_cache* c, int M, int offset, const int* 
         if (int rc = launch_qmm(m->h, uw.w, uw.s, uw.b, m->u, M, I, H, m->qmm_ws, m->qmm_ws_floats, st)) return rc;
         if (int rc = launch_silu_mul(m->g, m->u, m->a, static_cast<int64_t>(M) * I, st)) return rc;
       }
-      if (int rc = launch_qmm_epi_gm(QMM_RESIDUAL, m->a, L.p[SLOT_DOWN].wt, L.p[SLOT_DOWN].sbt, nullptr, nullptr, m->x,
-                                     m->x, M, H, I, m->qmm_ws, m->qmm_ws_floats, st))
-        return rc;
+      if (int rc = qmm_residual(m, m->a, L.p[SLOT_DOWN], M, st)) return rc;
     }
   }
   // ---- final norm, last row unless all logits, tied head (qwen3.rs:545-555) ----

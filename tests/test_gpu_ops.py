@@ -288,6 +288,39 @@ def test_qmm_vs_oracle(gpu, orc, M, N, K):
     assert _close(yb, orc.qmm_dequant(xb, wq, sb, bb), ulps=2, floor=1e-4) == 1.0
 
 
+# The few-rows GEMM: one row past the GEMV, edges of the 16-row tiles and of
+# their heights (48 | 49: 16 or 8 waves; 128 | 129: a second row tile), column
+# remainders of 64- and 128-column tiles, K of one slab, a broken last slab (2,
+# 6 and 18 groups), K split over workgroups, several rounds of workgroups
+SLAB = [(9, 64, 128), (16, 65, 384), (17, 100, 1152), (32, 1, 256), (33, 257, 2560), (48, 640, 9728), (49, 130, 640),
+        (65, 1000, 896), (80, 512, 5120), (112, 2560, 2560), (128, 192, 12288), (129, 96, 1152), (250, 520, 2560),
+        (300, 256, 4096), (24, 34000, 128), (57, 17000, 384), (130, 16390, 256)]
+
+
+@pytest.mark.parametrize("M,N,K", SLAB)
+def test_qmm_few_rows(gpu, orc, M, N, K):
+    import torch
+
+    print(f"qmm few rows M={M} N={N} K={K}", flush=True)
+    w, s, b = gpu.init_qlinear(7100 + M, N, K)
+    # the last row of x is the end of its allocation, y has guard rows
+    x = gpu.fill_normal_bf16(8100 + M, (M, K))
+    out = torch.full((M + 2, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    gpu.quantized_matmul(x, w, s, b, out=out[1:-1])
+    torch.cuda.synchronize()
+    assert (out[0] == 7.0).all() and (out[-1] == 7.0).all()
+    xb, wq, sb, bb = torch_bf16_bits(x), u32_of(w), torch_bf16_bits(s), torch_bf16_bits(b)
+    yb = torch_bf16_bits(out[1:-1])
+    assert _close(yb, orc.qmm_dequant(xb, wq, sb, bb), ulps=2, floor=1e-4) == 1.0
+    # scales and biases two bytes off a word take the tile kernel
+    if N * K <= 1 << 20:
+        so, bo = (torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape) for t in (s, b))
+        so.copy_(s)
+        bo.copy_(b)
+        yo = torch_bf16_bits(gpu.quantized_matmul(x, w, so, bo))
+        assert _close(yo, orc.qmm_dequant(xb, wq, sb, bb), ulps=2, floor=1e-4) == 1.0
+
+
 @pytest.mark.parametrize("M,N,K", [(64, 1024, 2560), (24, 768, 2048), (16, 2048, 4096), (5, 5120, 8192),
                                    (1, 4096, 2560)])
 def test_qmatmul_ws_matches_qmatmul(gpu, M, N, K):
