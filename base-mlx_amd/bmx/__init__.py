@@ -38,10 +38,16 @@ from ._lib import (  # noqa: F401
 IRWIN4_STD = 37837.226523565  # std of the sum of four uniform 16-bit integers
 
 
-def _torch():
-    import torch
+_T = None  # torch, imported by the first call that needs it
 
-    return torch
+
+def _torch():
+    global _T
+    if _T is None:
+        import torch
+
+        _T = torch
+    return _T
 
 
 def sigma_to_c(sigma: float) -> float:
@@ -52,14 +58,27 @@ def sigma_to_c(sigma: float) -> float:
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return t.data_ptr() if t is not None else None
+
+
+# The current stream's handle.  torch.cuda.current_stream() builds a Stream
+# object per call (most of a microsecond); its raw form is a plain int.  The
+# first call goes through the public function, which initialises the device.
+_raw_stream = None
 
 
 def _stream(stream=None):
+    global _raw_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is not None:
+        return _raw_stream()
     torch = _torch()
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    s = torch.cuda.current_stream().cuda_stream
+    get, dev = (getattr(torch._C, n, None) for n in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+    if get is not None and dev is not None:
+        _raw_stream = lambda: get(dev())  # noqa: E731
+    return s
 
 
 def _require_cuda(*ts):
@@ -71,17 +90,18 @@ def _require_cuda(*ts):
 
 
 def _qmatmul_args(x, w, scales, biases, group_size, bits):
-    torch = _torch()
+    bf16 = _torch().bfloat16
     _require_cuda(x, w, scales, biases)
-    if x.dtype != torch.bfloat16 or scales.dtype != torch.bfloat16 or biases.dtype != torch.bfloat16:
+    if x.dtype != bf16 or scales.dtype != bf16 or biases.dtype != bf16:
         raise BmxError(BMX_E_ARG, "x, scales and biases must be bfloat16")
-    K = x.shape[-1]
-    N = w.shape[0]
-    if bits == 4 and w.shape[-1] * 8 != K:
-        raise BmxError(BMX_E_SHAPE, f"w has {w.shape[-1]} words per row, K={K} needs {K // 8}")
-    if scales.shape != biases.shape or scales.shape[0] != N or scales.shape[-1] * group_size != K:
-        raise BmxError(BMX_E_SHAPE, f"scales/biases {tuple(scales.shape)} do not match N={N}, K={K}")
-    return x.numel() // K, N, K
+    xs, ws, ss = x.shape, w.shape, scales.shape
+    K = xs[-1]
+    N = ws[0]
+    if bits == 4 and ws[-1] * 8 != K:
+        raise BmxError(BMX_E_SHAPE, f"w has {ws[-1]} words per row, K={K} needs {K // 8}")
+    if ss != biases.shape or ss[0] != N or ss[-1] * group_size != K:
+        raise BmxError(BMX_E_SHAPE, f"scales/biases {tuple(ss)} do not match N={N}, K={K}")
+    return x.numel() // K, N, K, xs
 
 
 def quantized_matmul(x, w, scales, biases, transpose=True, group_size=64, bits=4, out=None, stream=None):
@@ -89,12 +109,11 @@ def quantized_matmul(x, w, scales, biases, transpose=True, group_size=64, bits=4
 
     transpose=False is rejected by the library (BMX_E_UNSUPPORTED), as the
     reference only ever passes True."""
-    torch = _torch()
-    M, N, K = _qmatmul_args(x, w, scales, biases, group_size, bits)
+    M, N, K, xs = _qmatmul_args(x, w, scales, biases, group_size, bits)
     if out is None:
-        out = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
-    call("bmx_qmatmul_affine", _ptr(x), _ptr(w), _ptr(scales), _ptr(biases), _ptr(out), M, N, K,
-         1 if transpose else 0, group_size, bits, _stream(stream))
+        out = x.new_empty((*xs[:-1], N))
+    call("bmx_qmatmul_affine", x.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), out.data_ptr(), M, N,
+         K, 1 if transpose else 0, group_size, bits, _stream(stream))
     return out
 
 
@@ -108,10 +127,9 @@ def quantized_matmul_ws(x, w, scales, biases, workspace, transpose=True, group_s
     """quantized_matmul with the split-K partials in `workspace` (a CUDA tensor
     of at least qmatmul_workspace_bytes(M, N, K) bytes, or None when that is
     0); never allocates device memory in the library."""
-    torch = _torch()
-    M, N, K = _qmatmul_args(x, w, scales, biases, group_size, bits)
+    M, N, K, xs = _qmatmul_args(x, w, scales, biases, group_size, bits)
     if out is None:
-        out = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
+        out = x.new_empty((*xs[:-1], N))
     wp, wb = (None, 0) if workspace is None else (_ptr(workspace), workspace.numel() * workspace.element_size())
     call("bmx_qmatmul_affine_ws", _ptr(x), _ptr(w), _ptr(scales), _ptr(biases), _ptr(out), M, N, K,
          1 if transpose else 0, group_size, bits, wp, wb, _stream(stream))
@@ -165,11 +183,10 @@ def fill_normal_bf16(seed: int, shape, sigma: float = 1.0, device="cuda", stream
 # ---------------------------------------------------------------------------
 def rms_norm(x, w, eps=1e-6, out=None, stream=None):
     """fast::rms_norm over the last axis (bf16)."""
-    torch = _torch()
     _require_cuda(x, w)
-    out = torch.empty_like(x) if out is None else out
+    out = _torch().empty_like(x) if out is None else out
     dim = x.shape[-1]
-    call("bmx_rms_norm", _ptr(x), _ptr(w), _ptr(out), x.numel() // dim, dim, ctypes.c_float(eps), _stream(stream))
+    call("bmx_rms_norm", x.data_ptr(), w.data_ptr(), out.data_ptr(), x.numel() // dim, dim, eps, _stream(stream))
     return out
 
 
@@ -179,7 +196,7 @@ def rope(x, theta, offset, out=None, stream=None):
     _require_cuda(x)
     H, T, D = x.shape
     out = torch.empty_like(x) if out is None else out
-    call("bmx_rope", _ptr(x), _ptr(out), H, T, D, ctypes.c_float(theta), offset, _stream(stream))
+    call("bmx_rope", _ptr(x), _ptr(out), H, T, D, theta, offset, _stream(stream))
     return out
 
 
@@ -206,7 +223,7 @@ def qk_norm_rope_kv(q, k, v, q_norm, k_norm, k_cache, v_cache, offset, eps=1e-6,
     Hq = q.shape[-1] // D
     q_out = torch.empty(Hq, M, D, dtype=torch.bfloat16, device=q.device)
     call("bmx_qk_norm_rope_kv", _ptr(q), _ptr(k), _ptr(v), _ptr(q_norm), _ptr(k_norm), _ptr(q_out), _ptr(k_cache),
-         _ptr(v_cache), M, Hq, Hkv, D, cap, offset, ctypes.c_float(eps), ctypes.c_float(theta), _stream(stream))
+         _ptr(v_cache), M, Hq, Hkv, D, cap, offset, eps, theta, _stream(stream))
     return q_out
 
 
@@ -222,7 +239,7 @@ def attention(q, k_cache, v_cache, offset, scale=None, use_workspace=True, works
         workspace = attention_workspace(Hq, M, q.device)
     nbytes = workspace.numel() * 4 if use_workspace else 0
     call("bmx_attention_gqa", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), Hq, Hkv, M, D, cap, offset,
-         ctypes.c_float(scale), _ptr(workspace if use_workspace else None), nbytes, _stream(stream))
+         scale, _ptr(workspace if use_workspace else None), nbytes, _stream(stream))
     return out
 
 
@@ -246,8 +263,8 @@ def qk_norm_rope_kv_attention(q, k, v, q_norm, k_norm, k_cache, v_cache, offset,
         workspace = attention_workspace(Hq, M, q.device)
     out = torch.empty(M, Hq * D, dtype=torch.bfloat16, device=q.device)
     call("bmx_qk_norm_rope_kv_attention", _ptr(q), _ptr(k), _ptr(v), _ptr(q_norm), _ptr(k_norm), _ptr(k_cache),
-         _ptr(v_cache), _ptr(out), M, Hq, Hkv, D, cap, offset, ctypes.c_float(eps), ctypes.c_float(theta),
-         ctypes.c_float(scale), _ptr(workspace), workspace.numel() * 4, _stream(stream))
+         _ptr(v_cache), _ptr(out), M, Hq, Hkv, D, cap, offset, eps, theta,
+         scale, _ptr(workspace), workspace.numel() * 4, _stream(stream))
     return out
 
 
@@ -308,7 +325,7 @@ def silu_mul(g, u, stream=None):
     torch = _torch()
     _require_cuda(g, u)
     y = torch.empty_like(g)
-    call("bmx_silu_mul", _ptr(g), _ptr(u), _ptr(y), g.numel(), _stream(stream))
+    call("bmx_silu_mul", g.data_ptr(), u.data_ptr(), y.data_ptr(), g.numel(), _stream(stream))
     return y
 
 
@@ -316,7 +333,7 @@ def add(a, b, stream=None):
     torch = _torch()
     _require_cuda(a, b)
     y = torch.empty_like(a)
-    call("bmx_add", _ptr(a), _ptr(b), _ptr(y), a.numel(), _stream(stream))
+    call("bmx_add", a.data_ptr(), b.data_ptr(), y.data_ptr(), a.numel(), _stream(stream))
     return y
 
 

@@ -108,6 +108,8 @@ SIGNATURES = {
 def load():
     """Load libbmx.so once and attach signatures; raise if it is not built."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -132,4 +134,7 @@ def check(rc: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args))
+    """One entry point; pointers and streams as plain ints (or None)."""
+    rc = getattr(_lib or load(), name)(*args)
+    if rc != 0:
+        raise BmxError(rc, last_error())

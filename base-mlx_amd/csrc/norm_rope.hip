@@ -21,10 +21,17 @@
 namespace bmx {
 
 RopeTable make_rope_table(int D, float theta) {
-  RopeTable t;
+  // 64 pow calls are most of a small call's host time: a thread keeps the
+  // table it made last (a function of D and theta alone)
+  thread_local int last_d = 0;
+  thread_local float last_theta = 0.0f;
+  thread_local RopeTable t;
+  if (D == last_d && theta == last_theta) return t;
   memset(&t, 0, sizeof(t));
   const int half = D / 2;
   for (int i = 0; i < half && i < 128; i++) t.inv_freq[i] = static_cast<float>(pow(static_cast<double>(theta), -static_cast<double>(i) / half));
+  last_d = D;
+  last_theta = theta;
   return t;
 }
 
