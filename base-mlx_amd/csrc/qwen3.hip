@@ -236,7 +236,8 @@ int forward_device(bmx_qwen3* m, bmx_kv_cache* c, int M, int offset, const int* 
   // long forwards norm and rotate q / k in the q|k|v GEMM's epilogue (the
   // attention then takes the flash kernel, which reads them from q_out and
   // the caches); the rotation's (cos, sin) once per forward
-  const bool rope_gemm = M > kRopeGemmMinM && hd == 128;
+  const bool few_qkv = qmm_few_rows(QMM_STORE, M, qd + 2 * kvd, H, true);
+  const bool rope_gemm = M > kRopeGemmMinM && hd == 128 && !few_qkv;
   if (rope_gemm) {
     if (int rc = launch_rope_cs(m->rope_cs, M, offset, pos_dev, m->rope, st)) return rc;
   }
@@ -269,13 +270,12 @@ int forward_device(bmx_qwen3* m, bmx_kv_cache* c, int M, int offset, const int* 
       uint16_t* y3[3] = {m->q, m->k, m->v};
       const int n3[3] = {qd, kvd, kvd};
       int rc = kNoFit;
-      const bool few = qmm_few_rows(QMM_STORE, M, qd + 2 * kvd, H, true);
-      if (rope_gemm && !few) {
+      if (rope_gemm) {
         const QkvRopeOut ro{L.q_norm, L.k_norm, m->qr, c->k(l), c->v(l), m->rope_cs, pos_dev, offset, c->cap, cf.eps};
         rc = launch_qmm_qkv_rope_gm(m->h, wt3, sb3, n3, M, H, ro, st);
         if (rc == BMX_OK) roped = true;
       }
-      if (rc == kNoFit && !few)
+      if (rc == kNoFit && !few_qkv)
         rc = launch_qmm_segments_gm(m->h, 3, wt3, sb3, y3, n3, M, H, m->qmm_ws, m->qmm_ws_floats, st);
       if (rc == kNoFit) {
         const uint32_t* w3[3] = {L.p[SLOT_Q].w, L.p[SLOT_K].w, L.p[SLOT_V].w};

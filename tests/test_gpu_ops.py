@@ -258,6 +258,61 @@ def test_argmax(gpu, orc, n):
     assert got[1] == 7 and got[2] == 0 and got[3] == 0
 
 
+@pytest.mark.parametrize("n", [8, 8200, 81928])
+def test_argmax_ties_nan_and_inf(gpu, orc, n):
+    """The 16-byte path's bookkeeping by unit: ties inside a unit and across
+    threads, -0 before +0, NaN anywhere, rows of NaN and -inf alone (first
+    -inf, else 0), the last unit, a row of +inf."""
+    nan, ninf = 0x7FC1, 0xFF80
+    rng = np.random.default_rng(n)
+    x = np.repeat(torch_bf16_bits(gpu.fill_normal_bf16(17, (1, n))), 9, axis=0).copy()
+    x[1, n - 1] = x[1, n - 3] = 0x4200  # 32.0 twice in the last unit
+    x[2, :] = np.where(rng.random(n) < 0.5, 0x8000, 0)
+    x[3, rng.random(n) < 0.3] = nan
+    x[4, :] = nan
+    x[4, n - 2:] = ninf
+    x[5, :] = nan
+    x[6, n // 2:] = 0x7F80
+    x[7, :] = ninf
+    x[7, 5] = nan
+    x[8, 3] = x[8, n - 8] = 0x4200
+    x[8, 0] = 0x7F81  # a signalling NaN beside them
+    f = bf16_to_f32(x)
+    want = np.where(np.isnan(f).all(axis=1), 0, np.argmax(np.where(np.isnan(f), -np.inf, f), axis=1))
+    for r in range(9):  # NaN counts as nothing, not as -inf
+        if not np.isnan(f[r]).all() and np.nanmax(f[r]) == -np.inf:
+            want[r] = int(np.flatnonzero(f[r] == -np.inf)[0])
+    np.testing.assert_array_equal(gpu.argmax_rows(to_torch_bf16(x)).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("n", [131072, 131080, 131064, 131073])
+def test_elementwise_vector_path(gpu, n):
+    """Either side of the 8-values-per-thread rule, and operands 2 bytes off a
+    16-byte address: the same bits each way; add in place."""
+    import torch
+
+    a = gpu.fill_normal_bf16(18, (n + 1,), sigma=3.0)
+    b = gpu.fill_normal_bf16(19, (n + 1,))
+    for op in (gpu.silu_mul, gpu.add):
+        one = torch_bf16_bits(op(a[1:], b[1:]))
+        two = torch_bf16_bits(op(a[1:].clone(), b[1:].clone()))
+        np.testing.assert_array_equal(one, two)
+    c = a[1:].clone()
+    gpu.call("bmx_add", c.data_ptr(), b[1:].data_ptr(), c.data_ptr(), n, gpu._stream())
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(torch_bf16_bits(c), torch_bf16_bits(a[1:] + b[1:]))
+
+
+@pytest.mark.parametrize("dim", [4096, 4104, 5120, 8192, 8200])
+def test_rms_norm_row_lengths(gpu, orc, dim):
+    x = gpu.fill_normal_bf16(20, (5, dim))
+    w = gpu.fill_normal_bf16(21, (dim,))
+    y = torch_bf16_bits(gpu.rms_norm(x, w))
+    # the sums' order may move bf16(x / rms) by one ulp, at most 2^-7 of it,
+    # which after the product with w is under two ulps of the result
+    assert np.max(bf16_ulp_diff(y, orc.rms_norm(torch_bf16_bits(x), torch_bf16_bits(w)))) <= 2
+
+
 def test_silu_mul_and_add(gpu, orc):
     g = gpu.fill_normal_bf16(15, (3, 9728), sigma=3.0)
     u = gpu.fill_normal_bf16(16, (3, 9728))
