@@ -38,25 +38,6 @@ namespace bmx {
 namespace {
 
 
-// LDS byte offset of a pointer into shared memory
-__device__ __forceinline__ uint32_t lds_offset(const void* p) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
-}
-// lane l's 16 (4) bytes at src go to LDS byte `dst` + 16 l (4 l); dst is
-// wave-uniform.  Waited for by vm_wait.  (One wait state between the write
-// of M0 and its use by an LDS load.)
-__device__ __forceinline__ void lds_load16(const void* src, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "memory");
-}
-__device__ __forceinline__ void lds_load4(const void* src, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(dst) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void vm_wait() {
-  static_assert(N >= 0 && N < 64, "vmcnt");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // waits until at most min(K, behind) slabs' loads (L each) are outstanding
 template <int K, int L>
 __device__ __forceinline__ void wait_behind(int behind) {

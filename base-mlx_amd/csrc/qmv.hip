@@ -1171,6 +1171,197 @@ __global__ void __launch_bounds__(kThreads) qmvp_kernel(const QmvParams p, const
   }
 }
 
+// Vocabulary projection of 2..8 rows of x.  qmvp_kernel reads a chunk of
+// every x row from LDS (64 bytes a lane and row) for each chunk of a weight
+// row: at 5 rows that is 5 LDS reads of 1 KB per 80 dot products, one wave
+// per SIMD, and it runs at LDS speed (151936 x 2560: 115 us, a third of the
+// VALU time).  Here a lane holds the same chunk of RPL weight rows, so one
+// read of x serves them all -- two; four rows measured 82 us against 77, a
+// third of the last round of tiles idle -- on two waves per SIMD.  At 2, 4, 5
+// and 8 rows of x: 67 -> 48, 97 -> 70, 114 -> 77, 172 -> 104 us.  W streams through a register ring of D chunks
+// that runs on into the next tile, and a tile's s and b go to LDS as they
+// lie in memory (global_load_lds), a tile ahead.  Every row is computed with
+// the operations of the other GEMV kernels in their order, the same S lanes
+// and chunk -> lane assignment, so its bits are theirs.
+constexpr int kRThreads = 512;
+
+template <int MT, int RPL, int D>
+__global__ void __launch_bounds__(kRThreads, 2) qmvr_kernel(const QmvParams p, const int S, const int ntiles) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int XU = 8;  // x units (8 values) per thread per staging batch
+  const int lshift = __builtin_ctz(S), slots = 64 >> lshift;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int slot = lane >> lshift, sl = lane & (S - 1);
+  const int M = p.m, K = p.K, G = K / 64, C = K / 32, W8 = K / 8, GU = G / 8;
+  const int NI = C >> lshift;               // chunks per lane and row (a multiple of D)
+  const int wr = slots * RPL, RB = 8 * wr;  // rows per wave, per workgroup
+  const int rows = p.seg[0].rows;
+  unsigned char* xs = smem;                                            // [MT][C] x 80 B
+  float* sxs = reinterpret_cast<float*>(smem + MT * C * kChunkBytes);  // [MT][C]
+  float* red = sxs + MT * C;                                           // [4][MT]
+  uint16_t* sbs = reinterpret_cast<uint16_t*>(red + 4 * MT);           // [2][s, b][RB][G]
+  const bool has_norm = p.norm_w != nullptr;
+
+  // ---- a tile's s and b: 16-byte pieces (8 groups of a row) in row order ----
+  const uint32_t sb0 = __builtin_amdgcn_readfirstlane(lds_offset(sbs));
+  const float rcp_gu = 1.0f / static_cast<float>(GU);
+  auto issue_sb = [&](int t, int buf) {
+    const int n = RB * GU / 64;  // instructions of 64 pieces per array
+    for (int i = wave; i < n; i += kRThreads / 64) {
+      const int pc = i * 64 + lane, r = udiv_small(pc, rcp_gu);
+      const int64_t off = static_cast<int64_t>(min(t * RB + r, rows - 1)) * G + (pc - r * GU) * 8;
+      const uint32_t at = __builtin_amdgcn_readfirstlane(sb0 + static_cast<uint32_t>(buf * 2) * RB * G * 2 + i * 1024);
+      lds_load16(p.seg[0].s + off, at);
+      lds_load16(p.seg[0].b + off, __builtin_amdgcn_readfirstlane(at + static_cast<uint32_t>(RB) * G * 2));
+    }
+  };
+  // ---- W ring: chunk u of the lane's rows of tile t ----
+  uint4 w[D][RPL];
+  auto issue_w = [&](int k, int t, int u) {
+    const int row0 = t * RB + wave * wr + slot;
+#pragma unroll
+    for (int j = 0; j < RPL; j++) {
+      const uint32_t* src = p.seg[0].w + static_cast<int64_t>(min(row0 + j * slots, rows - 1)) * (K / 8) +
+                            (sl + (u << lshift)) * 4;
+      const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src));
+      w[k][j] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+  };
+  int t = blockIdx.x;
+  issue_sb(t, 0);
+
+  // ---- x into LDS once, as qmvp_kernel stages it (the first 256 threads sum
+  // the squares, thread i units i, i + 256, ... of a row) ----
+  auto inv_of = [&](int m) { return gemv_norm_inv(red[m], red[MT + m], red[2 * MT + m], red[3 * MT + m], K, p.eps); };
+  if (has_norm) {
+    if (threadIdx.x < kThreads) {
+#pragma unroll
+      for (int m = 0; m < MT; m++) {
+        float ss = 0.0f;
+        if (m < M) {
+          for (int j = threadIdx.x; j < W8; j += kThreads)
+            ss = gemv_ss_unit(*reinterpret_cast<const uint4*>(p.x + m * p.ldx + j * 8), ss);
+        }
+        ss = lanes_sum(ss, 64);
+        if (lane == 0) red[wave * MT + m] = ss;
+      }
+    }
+    __syncthreads();
+  }
+  for (int b0 = 0; b0 < MT * W8; b0 += kRThreads * XU) {
+    uint4 xr[XU], nr[XU];
+#pragma unroll
+    for (int i = 0; i < XU; i++) {
+      const int idx = min(b0 + i * kRThreads + static_cast<int>(threadIdx.x), MT * W8 - 1);
+      const int m = idx / W8, j = idx - m * W8;
+      xr[i] = *reinterpret_cast<const uint4*>(p.x + min(m, M - 1) * p.ldx + j * 8);
+      nr[i] = *reinterpret_cast<const uint4*>((has_norm ? p.norm_w : p.x) + j * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < XU; i++) {
+      const int idx = b0 + i * kRThreads + static_cast<int>(threadIdx.x);
+      const bool act = idx < MT * W8;
+      const int m = act ? idx / W8 : 0, j = act ? idx - m * W8 : 0;
+      uint4 d = xr[i];
+      if (has_norm) d = gemv_norm_unit(d, nr[i], inv_of(m));
+      float part = act ? gemv_unit_sum(d) : 0.0f;
+      // a chunk of 32 values = 4 consecutive words = 4 consecutive lanes
+      part += dpp_f32<0xB1>(part);
+      part += dpp_f32<0x4E>(part);
+      if (act) {
+        *reinterpret_cast<uint4*>(xs + (m * C + (j >> 2)) * kChunkBytes + (j & 3) * 16) = permute_pairs(d);
+        if ((j & 3) == 0) sxs[m * C + (j >> 2)] = part;
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < D; k++) issue_w(k, t, k);
+  vm_wait<D * RPL>();  // the first tile's s and b
+  __syncthreads();
+
+  const NibbleK nk = nibble_consts();
+  const int g = static_cast<int>(gridDim.x);
+  for (int buf = 0; t < ntiles; t += g, buf ^= 1) {
+    const bool more = t + g < ntiles;
+    if (more) issue_sb(t + g, buf ^ 1);
+    const uint16_t* sl_ = sbs + buf * 2 * RB * G + (wave * wr + slot) * G;
+    float acc[RPL][MT];
+#pragma unroll
+    for (int j = 0; j < RPL; j++)
+#pragma unroll
+      for (int m = 0; m < MT; m++) acc[j][m] = 0.0f;
+    for (int u0 = 0; u0 < NI; u0 += D) {
+#pragma unroll
+      for (int k = 0; k < D; k++) {
+        const int u = u0 + k, c = sl + (u << lshift);
+        float sv[RPL], bb[RPL];
+#pragma unroll
+        for (int j = 0; j < RPL; j++) {
+          const uint16_t* a = sl_ + j * slots * G + (c >> 1);
+          gemv_sb(static_cast<uint32_t>(a[0]) | (static_cast<uint32_t>(a[RB * G]) << 16), sv[j], bb[j]);
+        }
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+          if (m >= M) break;
+          const uint4* xp = reinterpret_cast<const uint4*>(xs + (m * C + c) * kChunkBytes);
+          const uint4 x0 = xp[0], x1 = xp[1], x2 = xp[2], x3 = xp[3];
+          const float sx = sxs[m * C + c];
+#pragma unroll
+          for (int j = 0; j < RPL; j++)
+            acc[j][m] = gemv_chunk(w[k][j], x0, x1, x2, x3, sv[j], bb[j], sx, acc[j][m], nk);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // the chunk D on, in this tile or the next (past the last tile: this
+        // tile's again, never used)
+        const int un = u + D;
+        issue_w(k, un < NI || !more ? t : t + g, un < NI ? un : un - NI);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < RPL; j++) {
+      const int row = t * RB + wave * wr + j * slots + slot;
+#pragma unroll
+      for (int m = 0; m < MT; m++) acc[j][m] = lanes_sum(acc[j][m], S);
+      if (sl == 0 && row < rows) {
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+          if (m >= M) break;
+          gemv_store<QMV_STORE>(p, 0, m, rows, row, acc[j][m], acc[j][m]);
+        }
+      }
+    }
+    // the next tile's s and b are older than W loads already used, so they
+    // are in LDS; its buffer's last readers are past the last barrier
+    __syncthreads();
+  }
+}
+
+// Launches the row-blocked vocabulary GEMV when it applies (one segment,
+// plain store, whole rounds of chunks); kNoFit otherwise.
+template <int MT>
+int try_launch_qmvr(int S, const QmvParams& p, hipStream_t st) {
+  const int C = p.K / 32, G = p.K / 64;
+  if (!p.sb_vec || p.nseg != 1 || p.amax || C % S) return kNoFit;
+  const int ni = C / S, slots = 64 / S;
+  // two rows of x are near the memory rate either way; from 4096 columns on
+  // the kernels below are ahead (151936 x 4096: 64.1 against 69.0 us)
+  if (MT == 2 && ni > 10) return kNoFit;
+  constexpr int RPL = 2;
+  const int RB = 8 * slots * RPL;
+  if (RB * (G / 8) % 64 || RB * (G / 8) >= 1 << 20) return kNoFit;
+  const size_t lds = static_cast<size_t>(MT) * C * (kChunkBytes + 4) + 16ull * MT + 8ull * RB * G;
+  if (lds > 160 * 1024) return kNoFit;
+  const int ntiles = (p.seg[0].rows + RB - 1) / RB;
+  auto go = [&](auto kern) {
+    if (int rc = allow_lds(kern, lds)) return rc;
+    hipLaunchKernelGGL(kern, dim3(std::min(256, ntiles)), dim3(kRThreads), lds, st, p, S, ntiles);
+    return check_launch("qmvr");
+  };
+  if (ni % 5 == 0) return go(qmvr_kernel<MT, RPL, 5>);
+  if (ni % 4 == 0) return go(qmvr_kernel<MT, RPL, 4>);
+  return kNoFit;
+}
+
 template <int MT, int NI>
 int launch_qmvp_epi(QmvEpilogue epi, int S, const QmvParams& p, int ntiles, int grid, size_t lds, hipStream_t st) {
   // the vocabulary-sized projections are plain stores (the lm_head)
@@ -1327,6 +1518,13 @@ int launch_qmv(QmvParams p, QmvEpilogue epi, hipStream_t stream) {
   int rows_total = 0;
   for (int i = 0; i < p.nseg; i++) rows_total += p.seg[i].rows;
   const bool amax_multi = p.amax != nullptr && mt > 1;
+  if (rows_total >= kPersistentRows && mt > 1 && epi == QMV_STORE) {
+    const int rc = mt == 2   ? try_launch_qmvr<2>(S, p, stream)
+                   : mt == 4 ? try_launch_qmvr<4>(S, p, stream)
+                   : mt == 5 ? try_launch_qmvr<5>(S, p, stream)
+                             : try_launch_qmvr<8>(S, p, stream);
+    if (rc != kNoFit) return rc;
+  }
   if (rows_total >= kPersistentRows && !amax_multi) {
     const int rc = try_launch_qmvp(epi, mt, S, p, blocks, stream);
     if (rc != kNoFit) return rc;

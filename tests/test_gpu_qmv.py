@@ -153,3 +153,25 @@ def test_gemv_rows_independent_of_row_count(gpu, N, K):
         y = torch_bf16_bits(gpu.quantized_matmul(x[:M].contiguous(), w, s, b))
         for i in range(M):
             np.testing.assert_array_equal(y[i], singles[i][0], err_msg=f"M={M} row {i}")
+
+
+@pytest.mark.parametrize("N,K", [(65536, 512), (70001, 1024), (65600, 1536), (66000, 3072), (65537, 4096)])
+def test_vocabulary_gemv_rows_blocked(gpu, orc, N, K):
+    """The row-blocked vocabulary GEMV (2..8 rows; chunk rounds of 2 to 16 per
+    lane, tile remainders of 1 row up) has the bits of each row alone, and
+    sampled columns match the oracle."""
+    import torch
+
+    print(f"vocabulary rows N={N} K={K}", flush=True)
+    w, s, b = gpu.init_qlinear(4200 + N % 97, N, K)
+    x = gpu.fill_normal_bf16(4300 + K % 89, (8, K))
+    singles = torch.cat([gpu.quantized_matmul(x[i:i + 1], w, s, b) for i in range(8)])
+    cols = torch.cat([torch.arange(0, N, N // 150), torch.arange(N - 20, N)]).cuda()
+    ref = orc.qmatmul(torch_bf16_bits(x), u32_of(w[cols]), torch_bf16_bits(s[cols]), torch_bf16_bits(b[cols]))
+    for M in range(2, 9):
+        out = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        gpu.quantized_matmul(x[:M].contiguous(), w, s, b, out=out[:M])
+        assert torch.equal(out[:M], singles[:M]), M
+        assert (out[M] == 7.0).all()
+    frac, worst = _close_to_oracle(torch_bf16_bits(singles[:, cols]), ref)
+    assert frac == 1.0, worst
