@@ -439,6 +439,8 @@ class KvCache:
 class Qwen3:
     """Random-init Qwen3 on the GPU behind the C ABI (bmx_qwen3_*)."""
 
+    _held = (None, None)  # the last two outputs written from the model's own stream
+
     def __init__(self, cfg, seed, sigma=0.02, max_tokens=256):
         self.cfg = cfg
         h = ctypes.c_void_p()
@@ -492,8 +494,17 @@ class Qwen3:
         toks = np.ascontiguousarray(tokens, np.uint32)
         M = toks.size
         out = torch.empty(M if all_logits else 1, self.cfg.vocab, dtype=torch.bfloat16, device="cuda")
+        st = _stream(stream)
+        if not st:
+            # On the null stream the model works on a stream of its own, while
+            # torch would hand `out`, once dropped, to the next allocation of
+            # the null stream at once -- another model's logits, say, written
+            # from that model's stream.  A forward waits for the token upload
+            # of the one before it, which the stream runs after the one before
+            # that: so all but the last two outputs are complete.
+            self._held = (self._held[1], out)
         call("bmx_qwen3_forward", self.h, cache.h, toks.ctypes.data_as(ctypes.c_void_p), M, int(all_logits), _ptr(out),
-             _stream(stream))
+             st)
         return out if all_logits else out[0]
 
     def decode_step(self, cache, token, want_logits=False, stream=None):

@@ -390,3 +390,21 @@ def test_qmatmul_two_streams(gpu, orc):
         yb = bf16_to_f32(torch_bf16_bits(y)).astype(np.float64)
         r = bf16_to_f32(ref).astype(np.float64)
         assert np.mean(np.abs(yb - r) <= np.maximum(2 * np.abs(r) * 2.0 ** -7, 1e-3 * np.max(np.abs(r)))) > 0.999
+
+
+def test_forward_outputs_are_not_reused_in_flight(gpu):
+    """On the null stream each model writes its logits from a stream of its
+    own: a dropped output's memory must not become another model's output
+    while it may still be written."""
+    cfg = gpu.qwen3_config(256, 512, 2, 4, 2, vocab=1000)
+    a, b = gpu.Qwen3(cfg, 1, max_tokens=40), gpu.Qwen3(cfg, 2, max_tokens=40)
+    ca, cb = a.new_cache(64), b.new_cache(64)
+    toks = np.arange(40, dtype=np.uint32)
+    want = torch_bf16_bits(a.forward(ca, toks)).copy()
+    for _ in range(3):
+        ca.reset()
+        cb.reset()
+        dropped = b.forward(cb, toks).data_ptr()
+        got = a.forward(ca, toks)
+        assert got.data_ptr() != dropped
+        np.testing.assert_array_equal(torch_bf16_bits(got), want)
