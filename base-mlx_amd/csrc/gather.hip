@@ -165,10 +165,13 @@ __global__ void __launch_bounds__(kGThreads) gather_qmv_kernel(const GatherParam
 // read from memory by each lane through its own row pointer; B = the
 // nibbles as bf16 integers 128 + q, lane l holding W row l % 16.  The group
 // decomposition stays as in the per-route kernel, fp32 throughout:
-//   acc = fma(b - 128 s, Sx, fma(s, D, acc)) per group and output,
-// with Sx = x . 1 from one more product against a tile of ones, which puts
-// it in the accumulator's own layout.  Rows past the count repeat the last
-// row and are not stored; a row's result does not depend on its slot.
+//   acc = fma(s, D, acc) per group and output,
+//   acc += (b - 128 s) Sx over four groups on v_mfma_f32_16x16x4_f32,
+// with the group sums Sx taken once per workgroup while x is staged (pair
+// order, so a nibble pair is one v_and_or; against Sx by products with a tile
+// of ones in every wave and one FMA per output more, a third of the vector
+// instructions less).  Rows past the count repeat the last row and are not
+// stored; a row's result does not depend on its slot.
 //
 // What each operand needs decides where it comes from.  W is read once, so it
 // goes straight to registers: 16 bytes per lane and step of two groups (64
@@ -184,22 +187,19 @@ constexpr int kGXS = kGChunkK + 8;  // LDS row stride of x (odd number of 16-byt
 constexpr int kGWaves = 8, kGCols = 32 * kGWaves;  // waves and output columns per workgroup
 constexpr int gather_rows_sbstride(int K) { return (K / 128) | 1; }
 constexpr size_t gather_rows_lds(int mt, int K) {
-  return 2ull * 16 * mt * kGXS * 2 + 8ull * kGCols * gather_rows_sbstride(K);
+  return 2ull * 16 * mt * kGXS * 2 + 2ull * 16 * mt * 4 * 4 + 8ull * kGCols * gather_rows_sbstride(K);
 }
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
-// the 8 nibbles of a word, in order, as bf16 pairs 128 + q
+// the 8 nibbles of a word as bf16 128 + q, in the order of permute_pairs
 __device__ __forceinline__ bf16x8_t nibbles_bf16(uint32_t w, const NibbleK& k) {
-  // pair i: byte i of w under byte i of w >> 4 (one byte permute), then the
-  // low nibbles of both halves over the magic
-  const uint32_t h = w >> 4;
   uint4 r;
-  r.x = (__builtin_amdgcn_perm(h, w, 0x0c040c00u) & k.mask) | k.magic;
-  r.y = (__builtin_amdgcn_perm(h, w, 0x0c050c01u) & k.mask) | k.magic;
-  r.z = (__builtin_amdgcn_perm(h, w, 0x0c060c02u) & k.mask) | k.magic;
-  r.w = (__builtin_amdgcn_perm(h, w, 0x0c070c03u) & k.mask) | k.magic;
+  r.x = (w & k.mask) | k.magic;
+  r.y = ((w >> 4) & k.mask) | k.magic;
+  r.z = ((w >> 8) & k.mask) | k.magic;
+  r.w = ((w >> 12) & k.mask) | k.magic;
   return __builtin_bit_cast(bf16x8_t, r);
 }
 
@@ -210,7 +210,8 @@ __global__ void __launch_bounds__(64 * kGWaves, MT == 4 ? 2 : 4) gather_rows_ker
   constexpr int XU = 16 * MT * (kGChunkK / 8) / T;  // 16-byte units of an x chunk per thread
   extern __shared__ __align__(16) unsigned char smem[];
   uint16_t* xs = reinterpret_cast<uint16_t*>(smem);                             // [2][16 MT][kGXS]
-  uint2* sbs = reinterpret_cast<uint2*>(smem + 2 * 16 * MT * kGXS * 2);        // [kGCols][sbstride]: s pair, b pair
+  float* sxs = reinterpret_cast<float*>(smem + 2 * 16 * MT * kGXS * 2);         // [2][16 MT][4]: sums of a group
+  uint2* sbs = reinterpret_cast<uint2*>(sxs + 2 * 16 * MT * 4);                 // [kGCols][sbstride]: s pair, b pair
   __shared__ uint16_t list[kGList];
   __shared__ int wsum[kGWaves];
   const int K = p.K, S = K / 128, C = K / kGChunkK;
@@ -289,7 +290,6 @@ __global__ void __launch_bounds__(64 * kGWaves, MT == 4 ? 2 : 4) gather_rows_ker
     }
   }
   const NibbleK nk = nibble_consts();
-  const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
   const f32x4_t zero{0.0f, 0.0f, 0.0f, 0.0f};
 
   for (int w0 = 0; w0 < total; w0 += kGList) {
@@ -327,8 +327,11 @@ __global__ void __launch_bounds__(64 * kGWaves, MT == 4 ? 2 : 4) gather_rows_ker
       auto store_x = [&](int c) {
 #pragma unroll
         for (int k = 0; k < XU; k++) {
-          const int unit = tid + k * T;
-          *reinterpret_cast<uint4*>(xs + ((c & 1) * 16 * MT + unit / UR) * kGXS + (unit % UR) * 8) = xr[k];
+          const int unit = tid + k * T, row = (c & 1) * 16 * MT + unit / UR;
+          *reinterpret_cast<uint4*>(xs + row * kGXS + (unit % UR) * 8) = permute_pairs(xr[k]);
+          // a group is 8 units = 8 consecutive lanes
+          const float sum = lanes_sum(gemv_unit_sum(xr[k]), 8);
+          if ((unit & 7) == 0) sxs[row * 4 + (unit % UR) / 8] = sum;
         }
       };
       f32x4_t acc[MT][NT];
@@ -341,18 +344,17 @@ __global__ void __launch_bounds__(64 * kGWaves, MT == 4 ? 2 : 4) gather_rows_ker
         // of the second; after the swaps every lane holds words
         // 4 (q & 1) + 2 (q >> 1) + {0, 1} of each
         uint4 v[NT];
-        uint2 sb[NT];
+        uint32_t sw[NT];
 #pragma unroll
         for (int j = 0; j < NT; j++) {
           const auto a = __builtin_amdgcn_permlane32_swap(wr[u][j].x, wr[u][j].z, false, false);
           const auto b = __builtin_amdgcn_permlane32_swap(wr[u][j].y, wr[u][j].w, false, false);
           v[j] = make_uint4(a[0], b[0], a[1], b[1]);
-          sb[j] = sbs[((wave * NT + j) * 16 + li) * SB + c * D + u];
+          sw[j] = sbs[((wave * NT + j) * 16 + li) * SB + c * D + u].x;
         }
         const uint16_t* xt = xs + ((c & 1) * 16 * MT + li) * kGXS + u * 128 + (q & 1) * 32 + (q >> 1) * 16;
 #pragma unroll
         for (int g = 0; g < 2; g++) {
-          f32x4_t sx[MT];
           bf16x8_t xa[MT][2];
 #pragma unroll
           for (int i = 0; i < MT; i++) {
@@ -360,17 +362,10 @@ __global__ void __launch_bounds__(64 * kGWaves, MT == 4 ? 2 : 4) gather_rows_ker
             xa[i][1] = *reinterpret_cast<const bf16x8_t*>(xt + i * 16 * kGXS + g * 64 + 8);
           }
 #pragma unroll
-          for (int i = 0; i < MT; i++) {
-            sx[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][0], ones, zero, 0, 0, 0);
-            sx[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][1], ones, sx[i], 0, 0, 0);
-          }
-#pragma unroll
           for (int j = 0; j < NT; j++) {
             const bf16x8_t b0 = nibbles_bf16(g == 0 ? v[j].x : v[j].z, nk);
             const bf16x8_t b1 = nibbles_bf16(g == 0 ? v[j].y : v[j].w, nk);
-            const float sv = g == 0 ? __uint_as_float(sb[j].x << 16) : __uint_as_float(sb[j].x & 0xffff0000u);
-            const float bv = g == 0 ? __uint_as_float(sb[j].y << 16) : __uint_as_float(sb[j].y & 0xffff0000u);
-            const float bb = __builtin_fmaf(-128.0f, sv, bv);
+            const float sv = __uint_as_float(g == 0 ? sw[j] << 16 : sw[j] & 0xffff0000u);
             f32x4_t d[MT];
 #pragma unroll
             for (int i = 0; i < MT; i++) d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][0], b0, zero, 0, 0, 0);
@@ -379,9 +374,24 @@ __global__ void __launch_bounds__(64 * kGWaves, MT == 4 ? 2 : 4) gather_rows_ker
 #pragma unroll
             for (int i = 0; i < MT; i++)
 #pragma unroll
-              for (int r = 0; r < 4; r++)
-                acc[i][j][r] = __builtin_fmaf(bb, sx[i][r], __builtin_fmaf(sv, d[i][r], acc[i][j][r]));
+              for (int r = 0; r < 4; r++) acc[i][j][r] = __builtin_fmaf(sv, d[i][r], acc[i][j][r]);
           }
+        }
+      };
+      // + (b - 128 s) Sx of the chunk's four groups, lane (li, q): row li's
+      // sum and column li's factor of group q
+      auto bias = [&](int c) {
+        float sx[MT];
+#pragma unroll
+        for (int i = 0; i < MT; i++) sx[i] = sxs[((c & 1) * 16 * MT + i * 16 + li) * 4 + q];
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+          const uint2 sb = sbs[((wave * NT + j) * 16 + li) * SB + c * D + (q >> 1)];
+          const float sv = __uint_as_float((q & 1) ? sb.x & 0xffff0000u : sb.x << 16);
+          const float bv = __uint_as_float((q & 1) ? sb.y & 0xffff0000u : sb.y << 16);
+          const float bb = __builtin_fmaf(-128.0f, sv, bv);
+#pragma unroll
+          for (int i = 0; i < MT; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[i], bb, acc[i][j], 0, 0, 0);
         }
       };
       // chunk c + 1: x into registers at the top of chunk c, ahead of the W
@@ -403,6 +413,7 @@ __global__ void __launch_bounds__(64 * kGWaves, MT == 4 ? 2 : 4) gather_rows_ker
           __builtin_amdgcn_sched_barrier(0);
           load_w(u, cn * D + u);
         }
+        bias(c);
         // chunk c - 1's buffer: its reads ended before the last barrier
         store_x(c + 1);
         __syncthreads();
