@@ -324,7 +324,6 @@ int launch_epi(const QmmParams& p, const SlabPlan& s, hipStream_t stream) {
     case 12: return launch_one<EPI, 6, 64>(p, s, stream);
     case 13: return launch_one<EPI, 6, 128>(p, s, stream);
     case 14: return launch_one<EPI, 7, 64>(p, s, stream);
-    case 15: return launch_one<EPI, 7, 128>(p, s, stream);
     case 16: return launch_one<EPI, 8, 64>(p, s, stream);
     default: return launch_one<EPI, 8, 128>(p, s, stream);
   }
@@ -338,7 +337,7 @@ int launch_epi(const QmmParams& p, const SlabPlan& s, hipStream_t stream) {
 //     at 64; 151936 x 2560 141 -> 63 at 9, 133 -> 92 at 64;
 //   * more rows while the tiles are one round of the 256 CUs: 1024 x 2560
 //     18.2 -> 12.2 at 200 rows, 33.8 -> 22.1 at 2048; 12288 x 4096 55.7 ->
-//     50.0 at 200 (192 tiles); 4096 x 2560 42.8 -> 32.6 at 1024 (256 tiles),
+//     47 at 200 (192 tiles); 4096 x 2560 42.8 -> 32.6 at 1024 (256 tiles),
 //     but 55.1 -> 73 at 2048 (512 tiles);
 //   * 64 columns per tile (half the x reuse, but twice the CUs) where those
 //     tiles fit the round, with K split to fill it: 2560 x 9728 at 37 rows
@@ -355,6 +354,9 @@ SlabPlan slab_plan(QmmEpilogue epi, int M, int N, int K, int max_splits) {
   s.mt = (t16 + rt - 1) / rt;
   auto tiles = [&](int bn) { return (per * static_cast<int64_t>(N) + bn - 1) / bn * rt; };
   s.bn = tiles(64) <= 256 ? 64 : 128;
+  // 112-row tiles of 128 columns run slower than 128-row ones (12288 x 4096,
+  // 192 tiles: 224 rows 53.4 us, 256 rows 46.9; 64 columns: equal)
+  if (s.bn == 128 && s.mt == 7) s.mt = 8;
   const int step = s.mt <= 3 ? 8 : 4;  // whole slabs
   s.gps = (G + step - 1) / step * step;
   if (epi != QMM_SWIGLU && s.bn == 64) {

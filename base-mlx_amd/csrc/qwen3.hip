@@ -230,13 +230,16 @@ int forward_device(bmx_qwen3* m, bmx_kv_cache* c, int M, int offset, const int* 
   const int qd = nq * hd, kvd = nkv * hd;
   const float scale = 1.0f / sqrtf(static_cast<float>(hd));  // qwen3.rs:324
   const int L_max = pos_dev ? c->cap : offset + M;
-  if (M > 8 && m->gm_stale) {
+  // the group-major copies, unless every GEMM takes the few-rows kernel
+  const bool few_qkv = qmm_few_rows(QMM_STORE, M, qd + 2 * kvd, H, true);
+  if (M > 8 && m->gm_stale &&
+      !(few_qkv && qmm_few_rows(QMM_RESIDUAL, M, H, qd, false) && qmm_few_rows(QMM_SWIGLU, M, I, H, true) &&
+        qmm_few_rows(QMM_RESIDUAL, M, H, I, false))) {
     if (int rc = repack_prefill_weights(m, st)) return rc;
   }
   // long forwards norm and rotate q / k in the q|k|v GEMM's epilogue (the
   // attention then takes the flash kernel, which reads them from q_out and
   // the caches); the rotation's (cos, sin) once per forward
-  const bool few_qkv = qmm_few_rows(QMM_STORE, M, qd + 2 * kvd, H, true);
   const bool rope_gemm = M > kRopeGemmMinM && hd == 128 && !few_qkv;
   if (rope_gemm) {
     if (int rc = launch_rope_cs(m->rope_cs, M, offset, pos_dev, m->rope, st)) return rc;
