@@ -472,8 +472,9 @@ int launch_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* s, c
   GatherParams p{x, w, s, b, lhs, rhs, y, x_rstride, y_rstride, x_bcast, nxb, E, M, N, K, S, R};
   // From 1.25 routes per expert on, the expert's weights once for all of its
   // routes.  128 experts, gate|up 1536 x 2048 and down 2048 x 768, both
-  // calls: 128 routes 54.8 us per route, 54.2 by expert; 192 routes 76.5
-  // against 65; 800 routes 284 against 86; 2664 routes 843 against 160.
+  // calls, per route and by expert: 128 routes 54.8 and 54.9 us, 192 routes
+  // 76.5 and 76.3, 320 routes 116 and 85, 800 routes 284 and 85, 2664 routes
+  // 843 and 103.
   if (4ll * R >= 5ll * E && E <= 65535 && K % kGChunkK == 0 && aligned(s, 4) && aligned(b, 4) &&
       gather_rows_lds(4, K) <= 160 * 1024 - 4096 && static_cast<int64_t>(N) * (K / 8) <= UINT32_MAX) {
     // rows an expert gets on average decide the tile; more tiles than that
