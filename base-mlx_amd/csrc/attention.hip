@@ -1576,7 +1576,9 @@ int flash_split_blocks(int groups, int tiles, int tq, int Hq, int M, int offset,
   };
   int best = 0;
   double least = cost(most) * 0.9;  // a split has to promise 10%
-  for (int ns = 2; ns <= 64 && (most + ns - 1) / ns >= 2; ns++) {
+  // (no more than four workgroups per CU: the search stays a few thousand
+  // steps)
+  for (int ns = 2; ns <= 64 && (most + ns - 1) / ns >= 2 && static_cast<int64_t>(groups) * tiles * ns <= 4 * kCus; ns++) {
     const int bps = (most + ns - 1) / ns, n = (most + bps - 1) / bps;
     if (static_cast<size_t>(n) * Hq * M * (kD + 2) > part_floats) break;
     const double c = cost(bps);
