@@ -37,7 +37,6 @@
 namespace bmx {
 namespace {
 
-
 // waits until at most min(K, behind) slabs' loads (L each) are outstanding
 template <int K, int L>
 __device__ __forceinline__ void wait_behind(int behind) {
