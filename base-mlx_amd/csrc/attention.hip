@@ -1396,7 +1396,10 @@ __global__ void __launch_bounds__(256) attn_flash_merge_kernel(const AttnParams 
     }
 #pragma unroll
     for (int u = 0; u < B; u++) {
-      if (z0 + u >= ns || ml[u].x == -INFINITY) continue;  // no key of the split visible to the row
+      // no key of the split visible to the row (its O may hold 0 x NaN of
+      // hidden keys).  Scores that are all NaN leave m at -inf too, with l NaN:
+      // those go on, so the row comes out NaN as it does unsplit
+      if (z0 + u >= ns || (ml[u].x == -INFINITY && ml[u].y == 0.0f)) continue;
       const float mn = fmaxf(m, ml[u].x);
       const float wa = __builtin_amdgcn_exp2f(m - mn), wb = __builtin_amdgcn_exp2f(ml[u].x - mn);
       l = l * wa + ml[u].y * wb;

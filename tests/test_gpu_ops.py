@@ -146,6 +146,40 @@ def test_attention_flash_key_split(gpu, orc, Hq, Hkv, M, offset):
     np.testing.assert_array_equal(torch_bf16_bits(gpu.attention(q, kc, vc, offset, scale, workspace=small)), one)
 
 
+@pytest.mark.parametrize("Hq,Hkv,M,offset", [(32, 8, 70, 3000), (8, 8, 257, 1000)])
+def test_attention_flash_key_split_nan_and_inf(gpu, Hq, Hkv, M, offset):
+    """NaN and infinite scores come out of the split kernel where the unsplit
+    one has them, also where every score that a row has in a split is NaN (or
+    -inf: weight zero)."""
+    import torch
+
+    print(f"key split, NaN and inf: Hq={Hq} Hkv={Hkv} M={M} offset={offset}", flush=True)
+    nan, inf, rep, cap = float("nan"), float("inf"), Hq // Hkv, offset + M + 5
+    q = gpu.fill_normal_bf16(64, (Hq, M, 128))
+    kc = gpu.fill_normal_bf16(65, (Hkv, cap, 128))
+    vc = gpu.fill_normal_bf16(66, (Hkv, cap, 128))
+    q[0, 3, 17] = nan                        # a query: all its scores
+    kc[1, :offset // 2, 5] = nan             # half the keys of a head: whole splits
+    kc[2, offset // 2:offset, 5] = nan       # ... the other half
+    kc[3, offset - 1, 9] = nan               # one key
+    q[4 * rep:5 * rep] = q[4 * rep:5 * rep].abs().clamp(min=0.01)
+    kc[4, :offset // 2] = -inf               # scores of -inf over whole splits
+    q[5 * rep:6 * rep] = q[5 * rep:6 * rep].abs().clamp(min=0.01)
+    kc[5, offset // 2] = inf                 # a score of +inf
+    q[6 * rep:7 * rep] = q[6 * rep:7 * rep].abs().clamp(min=0.01)
+    kc[6] = -inf                             # nothing but -inf: zeros
+    one = gpu.attention(q, kc, vc, offset, use_workspace=False).float()
+    two = gpu.attention(q, kc, vc, offset, workspace=gpu.attention_workspace(Hq, 16)).float()
+    assert torch.equal(one.isnan(), two.isnan())
+    heads = one.isnan().view(M, Hq, 128)
+    assert heads[3, 0].all() and heads[:, rep:4 * rep].all() and heads[:, 5 * rep:6 * rep].all()
+    assert not heads[4:].any(dim=2)[:, :rep].any() and not heads[:, 4 * rep:5 * rep].any()
+    assert not one.view(M, Hq, 128)[:, 6 * rep:7 * rep].any()
+    # finite values: sums in another order, two bf16 roundings (2^-8 each) apart
+    fin = ~one.isnan()
+    assert ((one - two).abs()[fin] <= 2.0 ** -7 * one.abs()[fin] + 2e-3 * one[fin].abs().max()).all()
+
+
 def test_attention_workspace_reuse(gpu, orc):
     """One zero-filled workspace over calls of different split counts and row
     tilings: the arrival counters come back to zero after every call."""
