@@ -1317,6 +1317,11 @@ __global__ void __launch_bounds__(kRThreads, 2) qmvr_kernel(const QmvParams p, c
         issue_w(k, un < NI || !more ? t : t + g, un < NI ? un : un - NI);
       }
     }
+    // this wave's part of the next tile's s and b: newer than them are the D
+    // chunks of W in flight for that tile, and where a row is just D chunks
+    // (K = 1024) nothing else -- every chunk used above was requested before
+    // them, so no wait for W covers them
+    vm_wait<D * RPL>();
 #pragma unroll
     for (int j = 0; j < RPL; j++) {
       const int row = t * RB + wave * wr + j * slots + slot;
@@ -1330,8 +1335,8 @@ __global__ void __launch_bounds__(kRThreads, 2) qmvr_kernel(const QmvParams p, c
         }
       }
     }
-    // the next tile's s and b are older than W loads already used, so they
-    // are in LDS; its buffer's last readers are past the last barrier
+    // every wave's part of the next tile's s and b is in LDS; this tile's
+    // buffer has been read
     __syncthreads();
   }
 }

@@ -155,11 +155,14 @@ def test_gemv_rows_independent_of_row_count(gpu, N, K):
             np.testing.assert_array_equal(y[i], singles[i][0], err_msg=f"M={M} row {i}")
 
 
-@pytest.mark.parametrize("N,K", [(65536, 512), (70001, 1024), (65600, 1536), (66000, 3072), (65537, 4096)])
+@pytest.mark.parametrize("N,K", [(65536, 512), (70001, 1024), (65600, 1536), (66000, 3072), (65537, 4096),
+                                  (230001, 1024)])
 def test_vocabulary_gemv_rows_blocked(gpu, orc, N, K):
     """The row-blocked vocabulary GEMV (2..8 rows; chunk rounds of 2 to 16 per
     lane, tile remainders of 1 row up) has the bits of each row alone, and
-    sampled columns match the oracle."""
+    sampled columns match the oracle.  At K = 1024 a tile is one round of the
+    W ring, so only the explicit wait orders the next tile's scales and
+    biases (up to 8 tiles a workgroup at 230001 rows)."""
     import torch
 
     print(f"vocabulary rows N={N} K={K}", flush=True)
