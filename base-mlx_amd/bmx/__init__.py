@@ -439,7 +439,9 @@ class KvCache:
 class Qwen3:
     """Random-init Qwen3 on the GPU behind the C ABI (bmx_qwen3_*)."""
 
-    _held = (None, None)  # the last two outputs written from the model's own stream
+    # outputs written from the model's own stream that may still be written
+    # (at most two between calls)
+    _held = ()
 
     def __init__(self, cfg, seed, sigma=0.02, max_tokens=256):
         self.cfg = cfg
@@ -462,8 +464,9 @@ class Qwen3:
 
     def close(self):
         if self.h:
-            load().bmx_qwen3_destroy(self.h)
+            load().bmx_qwen3_destroy(self.h)  # waits for the device
             self.h = None
+            self._held = ()
 
     def __del__(self):
         try:
@@ -495,24 +498,32 @@ class Qwen3:
         M = toks.size
         out = torch.empty(M if all_logits else 1, self.cfg.vocab, dtype=torch.bfloat16, device="cuda")
         st = _stream(stream)
+        call("bmx_qwen3_forward", self.h, cache.h, toks.ctypes.data_as(ctypes.c_void_p), M, int(all_logits), _ptr(out),
+             st)
         if not st:
             # On the null stream the model works on a stream of its own, while
             # torch would hand `out`, once dropped, to the next allocation of
             # the null stream at once -- another model's logits, say, written
-            # from that model's stream.  A forward waits for the token upload
-            # of the one before it, which the stream runs after the one before
-            # that: so all but the last two outputs are complete.
-            self._held = (self._held[1], out)
-        call("bmx_qwen3_forward", self.h, cache.h, toks.ctypes.data_as(ctypes.c_void_p), M, int(all_logits), _ptr(out),
-             st)
+            # from that model's stream.  The call just made has waited for the
+            # token upload of the one before it, which the stream runs after
+            # the one before that: so all but the last two outputs are
+            # complete.  (Not before the call: until it has waited, and if it
+            # is refused, the older one may still be written.)
+            self._held = (*self._held[-1:], out)
         return out if all_logits else out[0]
+
+    def _waited(self, st):
+        """A call on stream `st` has returned that waits for its stream's end."""
+        if not st:
+            self._held = ()
 
     def decode_step(self, cache, token, want_logits=False, stream=None):
         torch = _torch()
         nxt = ctypes.c_uint32()
         out = torch.empty(self.cfg.vocab, dtype=torch.bfloat16, device="cuda") if want_logits else None
-        call("bmx_qwen3_decode_step", self.h, cache.h, ctypes.c_uint32(int(token)), ctypes.byref(nxt), _ptr(out),
-             _stream(stream))
+        st = _stream(stream)
+        call("bmx_qwen3_decode_step", self.h, cache.h, ctypes.c_uint32(int(token)), ctypes.byref(nxt), _ptr(out), st)
+        self._waited(st)
         return (nxt.value, out) if want_logits else nxt.value
 
     def generate_greedy(self, cache, prompt, max_new, eos=(151645, 151643), stream=None):
@@ -522,9 +533,10 @@ class Qwen3:
         e = np.ascontiguousarray(eos, np.uint32)
         out = np.empty(max_new, np.uint32)
         n = ctypes.c_int()
+        st = _stream(stream)
         call("bmx_generate_greedy", self.h, cache.h, p.ctypes.data_as(ctypes.c_void_p), p.size, max_new,
-             e.ctypes.data_as(ctypes.c_void_p), e.size, out.ctypes.data_as(ctypes.c_void_p), ctypes.byref(n),
-             _stream(stream))
+             e.ctypes.data_as(ctypes.c_void_p), e.size, out.ctypes.data_as(ctypes.c_void_p), ctypes.byref(n), st)
+        self._waited(st)
         return out[: n.value]
 
     def decode_greedy(self, cache, token, max_new, eos=(151645, 151643), stream=None):
