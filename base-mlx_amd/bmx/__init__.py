@@ -236,11 +236,24 @@ def attention(q, k_cache, v_cache, offset, scale=None, use_workspace=True, works
     scale = 1.0 / (D ** 0.5) if scale is None else scale
     out = torch.empty(M, Hq * D, dtype=torch.bfloat16, device=q.device)
     if use_workspace and workspace is None:
-        workspace = attention_workspace(Hq, M, q.device)
+        workspace = _call_workspace(Hq, M, q.device, stream)
     nbytes = workspace.numel() * 4 if use_workspace else 0
     call("bmx_attention_gqa", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), Hq, Hkv, M, D, cap, offset,
          scale, _ptr(workspace if use_workspace else None), nbytes, _stream(stream))
     return out
+
+
+def _call_workspace(Hq, M, device, stream):
+    """An attention workspace that lives for one call: allocated, cleared and
+    given back on the stream that uses it (torch hands memory dropped on one
+    stream to that stream's next allocation, whatever another still does)."""
+    if stream is None:
+        return attention_workspace(Hq, M, device)
+    torch = _torch()
+    if not isinstance(stream, torch.cuda.Stream):
+        stream = torch.cuda.ExternalStream(stream.cuda_stream, device=device)
+    with torch.cuda.stream(stream):
+        return attention_workspace(Hq, M, device)
 
 
 def attention_workspace(Hq, M, device="cuda"):
@@ -260,7 +273,7 @@ def qk_norm_rope_kv_attention(q, k, v, q_norm, k_norm, k_cache, v_cache, offset,
     Hq = q.shape[-1] // D
     scale = 1.0 / (D ** 0.5) if scale is None else scale
     if workspace is None:
-        workspace = attention_workspace(Hq, M, q.device)
+        workspace = _call_workspace(Hq, M, q.device, stream)
     out = torch.empty(M, Hq * D, dtype=torch.bfloat16, device=q.device)
     call("bmx_qk_norm_rope_kv_attention", _ptr(q), _ptr(k), _ptr(v), _ptr(q_norm), _ptr(k_norm), _ptr(k_cache),
          _ptr(v_cache), _ptr(out), M, Hq, Hkv, D, cap, offset, eps, theta,

@@ -96,3 +96,24 @@ def test_forward_on_a_given_stream_holds_nothing(fake):
     del out
     gc.collect()
     assert ref() is None
+
+
+def test_attention_workspace_of_a_call_belongs_to_its_stream(fake, monkeypatch):
+    """A call on a given stream allocates and clears its own workspace there:
+    freed on return, it goes to that stream's later allocations only.  (The
+    many-token path writes its key-split partials there too.)"""
+    made = []
+    monkeypatch.setattr(bmx, "_require_cuda", lambda *ts: None)
+    monkeypatch.setattr(bmx, "attention_workspace",
+                        lambda Hq, M, device: made.append(fake.current) or torch.zeros(8))
+    q, kc = torch.empty(8, 70, 128, dtype=torch.bfloat16), torch.empty(2, 80, 128, dtype=torch.bfloat16)
+    side = _Stream(64)
+    bmx.attention(q, kc, kc, 3, stream=side)
+    t, norm = torch.empty(1, 1024, dtype=torch.bfloat16), torch.empty(128, dtype=torch.bfloat16)
+    bmx.qk_norm_rope_kv_attention(t, t, t, norm, norm, kc, kc, 3, stream=side)
+    assert made == [side, side]
+    monkeypatch.setattr(bmx, "_stream", lambda s: 0)
+    bmx.attention(q, kc, kc, 3)
+    assert made[2] is fake.current
+    bmx.attention(q, kc, kc, 3, workspace=torch.zeros(8), stream=side)
+    assert len(made) == 3
