@@ -23,8 +23,10 @@
 // GEMV of qmv.hip stages them); each output row is served by S lanes that
 // stride over its 64-wide groups (32 bytes of W, one s and one b per group
 // and lane), with every W load of a lane issued before the staging.  With
-// more routes than experts, gather_rows_kernel (below) takes each expert's
+// many routes an expert, gather_rows_kernel (below) takes each expert's
 // routes together instead.
+#include <math.h>
+
 #include <algorithm>
 
 #include "bmx_device.h"
@@ -49,6 +51,7 @@ struct GatherParams {
   int x_bcast, nxb, E, M, N, K;  // nxb: x blocks
   int S;                // lanes per output row (power of two, 1..64)
   int R;                // routes
+  int run;              // by expert: tiles per unit
 };
 
 template <int MT>
@@ -157,13 +160,19 @@ __global__ void __launch_bounds__(kGThreads) gather_qmv_kernel(const GatherParam
 //
 // gather_qmv_kernel reads a route's whole weight matrix for that route
 // alone, so with R routes over E experts the same weights come from memory
-// (or the caches) R / E times.  Here a workgroup owns one expert and 128
-// output columns.  It finds the expert's routes by scanning the index array
-// (each thread a strip, one prefix sum; no scratch memory, no second
-// launch, so a captured graph replays with new routes), then multiplies
-// their rows in tiles of 16 MT on v_mfma_f32_16x16x32_bf16: A = x rows,
-// read from memory by each lane through its own row pointer; B = the
-// nibbles as bf16 integers 128 + q, lane l holding W row l % 16.  The group
+// (or the caches) R / E times.  Here a workgroup owns one unit -- a few tiles
+// of 16 MT rows of one expert -- and kGCols output columns.  The first E grid
+// rows are the experts' first units; the rows past them, as many as R routes
+// can need, take the further units of whichever experts have more: each
+// counts the routes of every expert (LDS counters) and finds its unit in the
+// prefix sum of those.  So an expert is spread over as many workgroups as it
+// has units, whatever share of the routes it takes (90% of 400 routes over
+// 128 experts to one of them, 1536 x 2048: 255 us where one workgroup walked
+// an expert's tiles, now 46), and workgroups without a unit end here.  No
+// scratch memory, no second launch: a captured graph replays with new routes.
+// The rows are multiplied
+// on v_mfma_f32_16x16x32_bf16: A = x rows (from LDS), B = the nibbles as bf16
+// integers 128 + q, lane l holding W row l % 16.  The group
 // decomposition stays as in the per-route kernel, fp32 throughout:
 //   acc = fma(s, D, acc) per group and output,
 //   acc += (b - 128 s) Sx over four groups on v_mfma_f32_16x16x4_f32,
@@ -181,10 +190,12 @@ __global__ void __launch_bounds__(kGThreads) gather_qmv_kernel(const GatherParam
 // per array and are staged whole.  (Read per lane and step instead, the 4-byte
 // s and b pieces and the x rows were 85% of the L1 misses, and the kernel ran
 // at the L2's rate: 226 MB of weights in 118 us.)
-constexpr int kGList = 1024;     // routes of the expert listed in LDS at a time
 constexpr int kGChunkK = 256;    // columns of x per LDS chunk
 constexpr int kGXS = kGChunkK + 8;  // LDS row stride of x (odd number of 16-byte units: no bank conflicts)
 constexpr int kGWaves = 8, kGCols = 32 * kGWaves;  // waves and output columns per workgroup
+constexpr int kGList = 1024;  // rows of a unit at most (their routes are listed in LDS)
+constexpr int kGMaxE = 4096;  // experts with a counter (in the LDS that holds x later)
+constexpr int kGFurther = 128;  // workgroups for units past the experts' first ones, about
 constexpr int gather_rows_sbstride(int K) { return (K / 128) | 1; }
 constexpr size_t gather_rows_lds(int mt, int K) {
   return 2ull * 16 * mt * kGXS * 2 + 2ull * 16 * mt * 4 * 4 + 8ull * kGCols * gather_rows_sbstride(K);
@@ -212,44 +223,91 @@ __global__ void __launch_bounds__(64 * kGWaves, MT == 4 ? 2 : 4) gather_rows_ker
   uint16_t* xs = reinterpret_cast<uint16_t*>(smem);                             // [2][16 MT][kGXS]
   float* sxs = reinterpret_cast<float*>(smem + 2 * 16 * MT * kGXS * 2);         // [2][16 MT][4]: sums of a group
   uint2* sbs = reinterpret_cast<uint2*>(sxs + 2 * 16 * MT * 4);                 // [kGCols][sbstride]: s pair, b pair
-  __shared__ uint16_t list[kGList];
+  __shared__ uint16_t list[kGList + 1];
   __shared__ int wsum[kGWaves];
+  __shared__ int unit_of[2];  // expert, unit of it
   const int K = p.K, S = K / 128, C = K / kGChunkK;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, q = lane >> 4;
-  const int e = blockIdx.y, n0 = blockIdx.x * kGCols;
-  // ---- this thread's part of the index array (every T-th): how many
-  // routes are e's, the first 32 of them as a bit mask ----
-  auto mine = [&](int r) {
-    return static_cast<int>(min(p.rhs ? p.rhs[r] : static_cast<uint32_t>(r), static_cast<uint32_t>(p.E - 1))) == e;
+  const int n0 = blockIdx.x * kGCols;
+  // ---- the experts of the routes; a thread's first ID (every T-th) stay in
+  // registers ----
+  constexpr int ID = 8;
+  auto expert_of = [&](int r) {
+    return static_cast<int>(min(p.rhs ? p.rhs[r] : static_cast<uint32_t>(r), static_cast<uint32_t>(p.E - 1)));
   };
-  int cnt = 0;
-  uint32_t mask = 0;
-  for (int i0 = 0; i0 * T < p.R; i0 += 4) {
-    bool hit[4];
+  int id[ID];
+  {
+    uint32_t v[ID];  // (every load issued before one is waited for)
 #pragma unroll
-    for (int u = 0; u < 4; u++) hit[u] = mine(min((i0 + u) * T + tid, p.R - 1));
+    for (int u = 0; u < ID; u++) v[u] = static_cast<uint32_t>(u * T + tid);
+    if (p.rhs) {
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const bool h = hit[u] && (i0 + u) * T + tid < p.R;
-      cnt += h;
-      if (i0 < 32) mask |= static_cast<uint32_t>(h) << (i0 + u);
+      for (int u = 0; u < ID; u++) v[u] = p.rhs[min(u * T + tid, p.R - 1)];
     }
-  }
-  int incl = cnt;
-  for (int off = 1; off < 64; off <<= 1) {
-    const int v = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += v;
-  }
-  if (lane == 63) wsum[wave] = incl;
-  __syncthreads();
-  int total = 0, before = incl - cnt;
 #pragma unroll
-  for (int w = 0; w < kGWaves; w++) {
-    if (w < wave) before += wsum[w];
-    total += wsum[w];
+    for (int u = 0; u < ID; u++)
+      id[u] = u * T + tid < p.R ? static_cast<int>(min(v[u], static_cast<uint32_t>(p.E - 1))) : -1;
   }
-  if (total == 0) return;  // uniform
+  // exclusive prefix sum over the workgroup's threads, and the total (a second
+  // use needs a barrier after the first)
+  int total = 0;
+  auto prefix = [&](int v) {
+    int incl = v;
+    for (int off = 1; off < 64; off <<= 1) {
+      const int w = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += w;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int before = incl - v;
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < kGWaves; w++) {
+      if (w < wave) before += wsum[w];
+      total += wsum[w];
+    }
+    return before;
+  };
+  // ---- this workgroup's unit: expert e, its rows from t0 on ----
+  const int UM = p.run * 16 * MT;  // rows of a unit
+  int e = blockIdx.y, t0 = 0;
+  if (e >= p.E) {  // a further unit: thread i owns experts i EP .. + EP - 1
+    int* counts = reinterpret_cast<int*>(smem);
+    for (int i = tid; i < p.E; i += T) counts[i] = 0;
+    if (tid == 0) unit_of[0] = -1;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < ID; u++)
+      if (id[u] >= 0) atomicAdd(&counts[id[u]], 1);
+    for (int r = ID * T + tid; r < p.R; r += T) atomicAdd(&counts[expert_of(r)], 1);
+    __syncthreads();
+    const int EP = (p.E + T - 1) / T, e0 = tid * EP, e1 = min(e0 + EP, p.E);
+    auto further = [&](int i) { return max(counts[i] * p.M - 1, 0) / UM; };
+    int mine = 0;
+    for (int i = e0; i < e1; i++) mine += further(i);
+    int at = e - p.E - prefix(mine);
+    if (at >= 0 && at < mine) {  // one thread, if any
+      int i = e0;
+      for (int n = further(i); at >= n; n = further(i)) {
+        at -= n;
+        i++;
+      }
+      unit_of[0] = i;
+      unit_of[1] = at + 1;
+    }
+    __syncthreads();
+    e = unit_of[0];
+    t0 = unit_of[1] * UM;
+    if (e < 0) return;  // uniform: no such unit
+  }
+  int cnt = 0;
+#pragma unroll
+  for (int u = 0; u < ID; u++) cnt += id[u] == e;
+  for (int r = ID * T + tid; r < p.R; r += T) cnt += expert_of(r) == e;
+  int idx = prefix(cnt);
+  const int rows = total * p.M;
+  if (rows == 0) return;  // uniform
 
   // ---- this wave's W rows (word offsets inside the expert) ----
   const uint32_t* we = p.w + static_cast<int64_t>(e) * p.N * (K / 8);
@@ -265,6 +323,23 @@ __global__ void __launch_bounds__(64 * kGWaves, MT == 4 ? 2 : 4) gather_rows_ker
 #pragma unroll
     for (int j = 0; j < NT; j++) wr[u][j] = *reinterpret_cast<const uint4*>(we + (wo[j] + step * 16));
   };
+  // ---- the unit's rows, t0 .. end - 1 of the expert's, as its routes first ..
+  // last in thread order ----
+  const int end = min(t0 + UM, rows), first = t0 / p.M, last = (end - 1) / p.M;
+  if (cnt > 0) {
+    idx -= first;
+    auto put = [&](int r) {
+      if (idx >= 0 && idx <= last - first) list[idx] = static_cast<uint16_t>(r);
+      idx++;
+    };
+#pragma unroll
+    for (int u = 0; u < ID; u++)
+      if (id[u] == e) put(u * T + tid);
+    for (int r = ID * T + tid; r < p.R; r += T)
+      if (expert_of(r) == e) put(r);
+  }
+  __syncthreads();
+
   // ---- s and b of the workgroup's columns (a contiguous block of each) ----
   const int SB = gather_rows_sbstride(K);
   {
@@ -292,154 +367,170 @@ __global__ void __launch_bounds__(64 * kGWaves, MT == 4 ? 2 : 4) gather_rows_ker
   const NibbleK nk = nibble_consts();
   const f32x4_t zero{0.0f, 0.0f, 0.0f, 0.0f};
 
-  for (int w0 = 0; w0 < total; w0 += kGList) {
-    // ---- routes w0 .. w0 + kGList - 1 of the expert (thread order) ----
-    __syncthreads();  // the last window's list has been read
-    if (cnt > 0) {
-      int idx = before - w0;
-      for (int i = 0; i * T + tid < p.R; i++)
-        if (i < 32 ? (mask >> i) & 1u : static_cast<uint32_t>(mine(i * T + tid))) {
-          if (idx >= 0 && idx < kGList) list[idx] = static_cast<uint16_t>(i * T + tid);
-          idx++;
-        }
+  for (int t = t0; t < end; t += 16 * MT) {
+    // this thread's part of an x chunk: 16-byte units tid + k T of
+    // [16 MT rows][kGChunkK / 8 units]
+    constexpr int UR = kGChunkK / 8;  // units per row
+    const uint16_t* xp[XU];
+#pragma unroll
+    for (int k = 0; k < XU; k++) {
+      const int unit = tid + k * T;
+      const int j = min(t + unit / UR, end - 1);
+      const int lr = p.M == 1 ? j : j / p.M, m = j - lr * p.M;
+      const int route = list[lr - first];
+      const int64_t xb = p.lhs ? min(p.lhs[route], static_cast<uint32_t>(p.nxb - 1)) : route / p.x_bcast;
+      xp[k] = p.x + xb * p.x_rstride + static_cast<int64_t>(m) * K + (unit % UR) * 8;
     }
-    __syncthreads();
-    const int rows = min(total - w0, kGList) * p.M;
-    for (int t = blockIdx.z * 16 * MT; t < rows; t += static_cast<int>(gridDim.z) * 16 * MT) {
-      // this thread's part of an x chunk: 16-byte units tid + k T of
-      // [16 MT rows][kGChunkK / 8 units]
-      constexpr int UR = kGChunkK / 8;  // units per row
-      const uint16_t* xp[XU];
+    uint4 xr[XU];
+    auto load_x = [&](int c) {
+#pragma unroll
+      for (int k = 0; k < XU; k++) xr[k] = *reinterpret_cast<const uint4*>(xp[k] + c * kGChunkK);
+    };
+    auto store_x = [&](int c) {
 #pragma unroll
       for (int k = 0; k < XU; k++) {
-        const int unit = tid + k * T;
-        const int j = min(t + unit / UR, rows - 1);
-        const int lr = p.M == 1 ? j : j / p.M, m = j - lr * p.M;
-        const int route = list[lr];
-        const int64_t xb = p.lhs ? min(p.lhs[route], static_cast<uint32_t>(p.nxb - 1)) : route / p.x_bcast;
-        xp[k] = p.x + xb * p.x_rstride + static_cast<int64_t>(m) * K + (unit % UR) * 8;
+        const int unit = tid + k * T, row = (c & 1) * 16 * MT + unit / UR;
+        *reinterpret_cast<uint4*>(xs + row * kGXS + (unit % UR) * 8) = permute_pairs(xr[k]);
+        // a group is 8 units = 8 consecutive lanes
+        const float sum = lanes_sum(gemv_unit_sum(xr[k]), 8);
+        if ((unit & 7) == 0) sxs[row * 4 + (unit % UR) / 8] = sum;
       }
-      uint4 xr[XU];
-      auto load_x = [&](int c) {
+    };
+    f32x4_t acc[MT][NT];
 #pragma unroll
-        for (int k = 0; k < XU; k++) xr[k] = *reinterpret_cast<const uint4*>(xp[k] + c * kGChunkK);
-      };
-      auto store_x = [&](int c) {
+    for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int k = 0; k < XU; k++) {
-          const int unit = tid + k * T, row = (c & 1) * 16 * MT + unit / UR;
-          *reinterpret_cast<uint4*>(xs + row * kGXS + (unit % UR) * 8) = permute_pairs(xr[k]);
-          // a group is 8 units = 8 consecutive lanes
-          const float sum = lanes_sum(gemv_unit_sum(xr[k]), 8);
-          if ((unit & 7) == 0) sxs[row * 4 + (unit % UR) / 8] = sum;
+      for (int j = 0; j < NT; j++) acc[i][j] = zero;
+    auto compute = [&](int u, int c) {
+      // lanes q 0, 1 hold a row's 8 words of the step's first group, q 2, 3
+      // of the second; after the swaps every lane holds words
+      // 4 (q & 1) + 2 (q >> 1) + {0, 1} of each
+      uint4 v[NT];
+      uint32_t sw[NT];
+#pragma unroll
+      for (int j = 0; j < NT; j++) {
+        const auto a = __builtin_amdgcn_permlane32_swap(wr[u][j].x, wr[u][j].z, false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(wr[u][j].y, wr[u][j].w, false, false);
+        v[j] = make_uint4(a[0], b[0], a[1], b[1]);
+        sw[j] = sbs[((wave * NT + j) * 16 + li) * SB + c * D + u].x;
+      }
+      const uint16_t* xt = xs + ((c & 1) * 16 * MT + li) * kGXS + u * 128 + (q & 1) * 32 + (q >> 1) * 16;
+#pragma unroll
+      for (int g = 0; g < 2; g++) {
+        bf16x8_t xa[MT][2];
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+          xa[i][0] = *reinterpret_cast<const bf16x8_t*>(xt + i * 16 * kGXS + g * 64);
+          xa[i][1] = *reinterpret_cast<const bf16x8_t*>(xt + i * 16 * kGXS + g * 64 + 8);
         }
-      };
-      f32x4_t acc[MT][NT];
-#pragma unroll
-      for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int j = 0; j < NT; j++) acc[i][j] = zero;
-      auto compute = [&](int u, int c) {
-        // lanes q 0, 1 hold a row's 8 words of the step's first group, q 2, 3
-        // of the second; after the swaps every lane holds words
-        // 4 (q & 1) + 2 (q >> 1) + {0, 1} of each
-        uint4 v[NT];
-        uint32_t sw[NT];
 #pragma unroll
         for (int j = 0; j < NT; j++) {
-          const auto a = __builtin_amdgcn_permlane32_swap(wr[u][j].x, wr[u][j].z, false, false);
-          const auto b = __builtin_amdgcn_permlane32_swap(wr[u][j].y, wr[u][j].w, false, false);
-          v[j] = make_uint4(a[0], b[0], a[1], b[1]);
-          sw[j] = sbs[((wave * NT + j) * 16 + li) * SB + c * D + u].x;
+          const bf16x8_t b0 = nibbles_bf16(g == 0 ? v[j].x : v[j].z, nk);
+          const bf16x8_t b1 = nibbles_bf16(g == 0 ? v[j].y : v[j].w, nk);
+          const float sv = __uint_as_float(g == 0 ? sw[j] << 16 : sw[j] & 0xffff0000u);
+          f32x4_t d[MT];
+#pragma unroll
+          for (int i = 0; i < MT; i++) d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][0], b0, zero, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < MT; i++) d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][1], b1, d[i], 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[i][j][r] = __builtin_fmaf(sv, d[i][r], acc[i][j][r]);
         }
-        const uint16_t* xt = xs + ((c & 1) * 16 * MT + li) * kGXS + u * 128 + (q & 1) * 32 + (q >> 1) * 16;
+      }
+    };
+    // + (b - 128 s) Sx of the chunk's four groups, lane (li, q): row li's
+    // sum and column li's factor of group q
+    auto bias = [&](int c) {
+      float sx[MT];
 #pragma unroll
-        for (int g = 0; g < 2; g++) {
-          bf16x8_t xa[MT][2];
+      for (int i = 0; i < MT; i++) sx[i] = sxs[((c & 1) * 16 * MT + i * 16 + li) * 4 + q];
 #pragma unroll
-          for (int i = 0; i < MT; i++) {
-            xa[i][0] = *reinterpret_cast<const bf16x8_t*>(xt + i * 16 * kGXS + g * 64);
-            xa[i][1] = *reinterpret_cast<const bf16x8_t*>(xt + i * 16 * kGXS + g * 64 + 8);
-          }
+      for (int j = 0; j < NT; j++) {
+        const uint2 sb = sbs[((wave * NT + j) * 16 + li) * SB + c * D + (q >> 1)];
+        const float sv = __uint_as_float((q & 1) ? sb.x & 0xffff0000u : sb.x << 16);
+        const float bv = __uint_as_float((q & 1) ? sb.y & 0xffff0000u : sb.y << 16);
+        const float bb = __builtin_fmaf(-128.0f, sv, bv);
 #pragma unroll
-          for (int j = 0; j < NT; j++) {
-            const bf16x8_t b0 = nibbles_bf16(g == 0 ? v[j].x : v[j].z, nk);
-            const bf16x8_t b1 = nibbles_bf16(g == 0 ? v[j].y : v[j].w, nk);
-            const float sv = __uint_as_float(g == 0 ? sw[j] << 16 : sw[j] & 0xffff0000u);
-            f32x4_t d[MT];
+        for (int i = 0; i < MT; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[i], bb, acc[i][j], 0, 0, 0);
+      }
+    };
+    // chunk c + 1: x into registers at the top of chunk c, ahead of the W
+    // loads of its steps (loads complete in order, so the x stores at the
+    // bottom leave those in flight), each W step into the registers the
+    // step before it freed.  Loads past the last chunk repeat it.
+    load_x(0);
 #pragma unroll
-            for (int i = 0; i < MT; i++) d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][0], b0, zero, 0, 0, 0);
+    for (int u = 0; u < D; u++) load_w(u, u);
+    store_x(0);
+    __syncthreads();
+    for (int c = 0; c < C; c++) {
+      const int cn = min(c + 1, C - 1);
+      load_x(cn);
 #pragma unroll
-            for (int i = 0; i < MT; i++) d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][1], b1, d[i], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < MT; i++)
-#pragma unroll
-              for (int r = 0; r < 4; r++) acc[i][j][r] = __builtin_fmaf(sv, d[i][r], acc[i][j][r]);
-          }
-        }
-      };
-      // + (b - 128 s) Sx of the chunk's four groups, lane (li, q): row li's
-      // sum and column li's factor of group q
-      auto bias = [&](int c) {
-        float sx[MT];
-#pragma unroll
-        for (int i = 0; i < MT; i++) sx[i] = sxs[((c & 1) * 16 * MT + i * 16 + li) * 4 + q];
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-          const uint2 sb = sbs[((wave * NT + j) * 16 + li) * SB + c * D + (q >> 1)];
-          const float sv = __uint_as_float((q & 1) ? sb.x & 0xffff0000u : sb.x << 16);
-          const float bv = __uint_as_float((q & 1) ? sb.y & 0xffff0000u : sb.y << 16);
-          const float bb = __builtin_fmaf(-128.0f, sv, bv);
-#pragma unroll
-          for (int i = 0; i < MT; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[i], bb, acc[i][j], 0, 0, 0);
-        }
-      };
-      // chunk c + 1: x into registers at the top of chunk c, ahead of the W
-      // loads of its steps (loads complete in order, so the x stores at the
-      // bottom leave those in flight), each W step into the registers the
-      // step before it freed.  Loads past the last chunk repeat it.
-      load_x(0);
-#pragma unroll
-      for (int u = 0; u < D; u++) load_w(u, u);
-      store_x(0);
+      for (int u = 0; u < D; u++) {
+        __builtin_amdgcn_sched_barrier(0);
+        compute(u, c);
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(u, cn * D + u);
+      }
+      bias(c);
+      // chunk c - 1's buffer: its reads ended before the last barrier
+      store_x(c + 1);
       __syncthreads();
-      for (int c = 0; c < C; c++) {
-        const int cn = min(c + 1, C - 1);
-        load_x(cn);
-#pragma unroll
-        for (int u = 0; u < D; u++) {
-          __builtin_amdgcn_sched_barrier(0);
-          compute(u, c);
-          __builtin_amdgcn_sched_barrier(0);
-          load_w(u, cn * D + u);
-        }
-        bias(c);
-        // chunk c - 1's buffer: its reads ended before the last barrier
-        store_x(c + 1);
-        __syncthreads();
-      }
-#pragma unroll
-      for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int j = t + i * 16 + 4 * q + r;
-          if (j >= rows) continue;
-          const int lr = p.M == 1 ? j : j / p.M, m = j - lr * p.M;
-          uint16_t* yr = p.y + static_cast<int64_t>(list[lr]) * p.y_rstride + static_cast<int64_t>(m) * p.N;
-#pragma unroll
-          for (int k = 0; k < NT; k++)
-            if (n[k] < p.N) yr[n[k]] = f2bf(acc[i][k][r]);
-        }
     }
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int j = t + i * 16 + 4 * q + r;
+        if (j >= end) continue;
+        const int lr = p.M == 1 ? j : j / p.M, m = j - lr * p.M;
+        uint16_t* yr = p.y + static_cast<int64_t>(list[lr - first]) * p.y_rstride + static_cast<int64_t>(m) * p.N;
+#pragma unroll
+        for (int k = 0; k < NT; k++)
+          if (n[k] < p.N) yr[n[k]] = f2bf(acc[i][k][r]);
+      }
   }
 }
 
+// units past the experts' first ones that R routes of M rows can make
+int64_t gather_rows_further(int unit_rows, int M, int R) { return static_cast<int64_t>(R) * M / unit_rows; }
+
+// Whether the routes of an expert are better multiplied together, from what
+// both kernels take (us; 1 to 128 experts, 1 to 50 routes each, 200 x 256 to
+// 14336 x 4096, 1 to 8 rows a route): per route every route's weights at the
+// caches' rate, and each expert's once from memory; by expert the chain of K
+// chunks that a workgroup walks, or each expert's weights once from memory.
+// 1536 x 2048, per route and by expert: 8 experts 16 routes 7.6 and 16.6, 80
+// routes 18.9 and 17.4; 32 experts 40 routes 16.7 and 18.3; 128 experts 160
+// routes 40.7 and 34.6, 1280 routes 259 and 58.  It picks the slower one by
+// more than 5% only near the line: at most 10% (1.4 us) over those shapes.
+bool gather_by_expert(int E, int M, int N, int K, int R) {
+  const double mb = static_cast<double>(N) * K * 0.5625e-6, used = mb * E * (1.0 - exp(-static_cast<double>(R) / E));
+  const double per_route = 3.7 + M * (0.2 + 0.35 * K / 1024.0) + R * (0.005 + (1.0 + 0.4 * (M - 1)) * mb / 9.5) +
+                           used / 16.0;
+  const double chain = 5.5 + 5.1 * K / 1024.0, by_expert = std::max(chain, 0.4 * chain + used / 4.3);
+  return 1.06 * by_expert < per_route;
+}
+
 template <int MT>
-int launch_gather_rows(const GatherParams& p, int64_t avg, hipStream_t stream) {
+int launch_gather_rows(GatherParams p, hipStream_t stream) {
   const size_t lds = gather_rows_lds(MT, p.K);
   if (int rc = allow_lds(gather_rows_kernel<MT>, lds)) return rc;
-  const dim3 grid((p.N + kGCols - 1) / kGCols, p.E,
-                  static_cast<unsigned>(std::min<int64_t>((avg + 16 * MT - 1) / (16 * MT), 64)));
+  const int cols = (p.N + kGCols - 1) / kGCols;
+  // Tiles per unit: one where the CUs hold every unit there can be; else so
+  // many that the further units are few, since an even routing leaves them
+  // nothing to do (2664 routes over 128 experts, 1536 x 2048 and 2048 x 768:
+  // 122 us with one tile a unit, 112 so; with 90% of the routes to one expert
+  // the first takes 90 us so and 136, of 1125 with an expert to a workgroup)
+  const int64_t most = gather_rows_further(16 * MT, p.M, p.R), rows = std::max(1, kGFurther / cols);
+  p.run = 1;
+  if (cols * (std::min(p.E, p.R) + most) > 256)
+    p.run = static_cast<int>(std::min<int64_t>((most + rows - 1) / rows, kGList / (16 * MT)));
+  if (p.run < 1) p.run = 1;
+  const dim3 grid(cols, p.E + static_cast<unsigned>(gather_rows_further(p.run * 16 * MT, p.M, p.R)));
   hipLaunchKernelGGL(gather_rows_kernel<MT>, grid, dim3(64 * kGWaves), lds, stream, p);
   return check_launch("gather_qmm rows");
 }
@@ -469,21 +560,21 @@ int launch_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* s, c
   const size_t lds = static_cast<size_t>(mt) * (K / 32) * (kGChunk + 4);
   if (lds > 160 * 1024) return set_error(BMX_E_UNSUPPORTED, "gather_qmm: M*K=%d too large", M * K);
   const int rb = 4 * (64 / S);
-  GatherParams p{x, w, s, b, lhs, rhs, y, x_rstride, y_rstride, x_bcast, nxb, E, M, N, K, S, R};
-  // From 1.25 routes per expert on, the expert's weights once for all of its
-  // routes.  128 experts, gate|up 1536 x 2048 and down 2048 x 768, both
-  // calls, per route and by expert: 128 routes 54.8 and 54.9 us, 192 routes
-  // 76.5 and 76.3, 320 routes 116 and 85, 800 routes 284 and 85, 2664 routes
-  // 843 and 103.
-  if (4ll * R >= 5ll * E && E <= 65535 && K % kGChunkK == 0 && aligned(s, 4) && aligned(b, 4) &&
-      gather_rows_lds(4, K) <= 160 * 1024 - 4096 && static_cast<int64_t>(N) * (K / 8) <= UINT32_MAX) {
-    // rows an expert gets on average decide the tile; more tiles than that
-    // are walked by the same workgroup
+  GatherParams p{x, w, s, b, lhs, rhs, y, x_rstride, y_rstride, x_bcast, nxb, E, M, N, K, S, R, 1};
+  if (E <= kGMaxE && K % kGChunkK == 0 && aligned(s, 4) && aligned(b, 4) &&
+      gather_rows_lds(4, K) <= 160 * 1024 - 4096 && static_cast<int64_t>(N) * (K / 8) <= UINT32_MAX &&
+      gather_by_expert(E, M, N, K, R)) {
+    // the rows an expert gets on average decide the tile; shorter ones where
+    // those leave CUs idle too (1536 x 2048, 8 experts, 400 routes: 32 rows
+    // 20.8 us, 16 rows 17.8; 32 experts, 640 routes, 420 workgroups of 16
+    // rows: 23.3 and 30.6)
     const int64_t rows = static_cast<int64_t>(R) * M;
-    const int64_t avg = (rows + E - 1) / E;
-    return avg <= 8    ? launch_gather_rows<1>(p, avg, stream)
-           : avg <= 48 ? launch_gather_rows<2>(p, avg, stream)
-                       : launch_gather_rows<4>(p, avg, stream);
+    const int64_t avg = (rows + E - 1) / E, cols = (N + kGCols - 1) / kGCols;
+    int t = avg <= 8 ? 1 : avg <= 48 ? 2 : 4;
+    while (t > 1 && cols * (std::min(E, R) + gather_rows_further(8 * t, M, R)) <= 256) t /= 2;
+    return t == 1   ? launch_gather_rows<1>(p, stream)
+           : t == 2 ? launch_gather_rows<2>(p, stream)
+                    : launch_gather_rows<4>(p, stream);
   }
   const dim3 grid((N + rb - 1) / rb, R);
   const void* kern = mt == 1   ? reinterpret_cast<const void*>(gather_qmv_kernel<1>)

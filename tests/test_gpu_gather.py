@@ -135,15 +135,21 @@ def test_gather_qmm_indexed_errors(gpu):
         assert ei.value.code == code, kw
 
 
-# From 1.25 routes per expert on, one workgroup multiplies all of an expert's
-# routes (16, 32 or 64 rows a tile, by the average): (E, N, K, M, R, x_bcast,
-# skew); skew sends that share of the routes to expert 1.  Column remainders
-# (N 100, 257), one and several 256-column chunks, rows per route that
-# straddle tiles, an expert above the 1024 routes listed at a time, index
-# arrays beyond the 16384 entries kept as bits, experts without a route.
+# Where that is faster, an expert's routes are multiplied together, in units of
+# 16, 32 or 64 rows (by the average, and 256 workgroups): (E, N, K, M, R,
+# x_bcast, skew); skew sends that share of the routes to expert 1.  Column
+# remainders (N 100, 257), one and several 256-column chunks, rows per route
+# that straddle tiles, an expert above 1024 routes, index arrays beyond the
+# 4096 entries kept in registers, experts without a route.
 ROWS = [(4, 100, 256, 1, 5, 1, 0.0), (16, 257, 768, 1, 40, 8, 0.0), (6, 96, 512, 3, 33, 3, 0.5),
         (3, 64, 256, 8, 60, 1, 0.9), (5, 288, 512, 1, 200, 4, 0.3), (2, 32, 256, 1, 2500, 1, 0.99),
         (4, 40, 256, 1, 20011, 1, 0.25), (9, 256, 2048, 1, 300, 1, 0.0)]
+# ... 16 rows a unit over 8 chunks, even and all but one route to one expert;
+# 32 rows over 3 chunks; 64 rows over 8, 3 and 2 chunks with 1, 2 and 3 rows a
+# route; more experts than threads, and the most there are counters for
+ROWS += [(8, 1536, 2048, 1, 160, 8, 0.0), (16, 1200, 2048, 1, 200, 1, 0.99), (32, 1000, 768, 1, 1200, 8, 0.3),
+         (3, 1500, 2048, 1, 1500, 1, 0.3), (4, 1030, 768, 2, 1000, 1, 0.6), (4, 1030, 512, 3, 700, 1, 0.3),
+         (600, 64, 256, 1, 1500, 1, 0.1), (4096, 32, 256, 1, 9000, 1, 0.05)]
 
 
 @pytest.mark.parametrize("E,N,K,M,R,x_bcast,skew", ROWS)
@@ -171,3 +177,18 @@ def test_gather_qmm_by_expert(gpu, orc, E, N, K, M, R, x_bcast, skew):
     np.testing.assert_array_equal(torch_bf16_bits(z)[1:], torch_bf16_bits(y)[perm[1:]])
     last = orc.gather_qmm(torch_bf16_bits(x)[lhs[:1]], wq, sq, bq, np.array([E - 1], np.uint32), 1)
     assert _close(torch_bf16_bits(z)[:1], last) > 0.999
+
+
+@pytest.mark.parametrize("E,N,K,M,R", [(8, 1536, 2048, 1, 16), (1, 2048, 768, 1, 2), (4, 512, 512, 2, 8)])
+def test_gather_qmm_few_routes_stay_apart(gpu, orc, E, N, K, M, R):
+    """Few routes over few experts leave CUs idle when taken by expert, so
+    they have the bits of the per-route kernel: those of the same routes among
+    enough further experts that no expert could get two."""
+    import torch
+
+    (w, s, b), _ = _experts(gpu, orc, 6000 + K, E, N, K)
+    more = [torch.cat([t] + [t[:1]] * (2 * R)).contiguous() for t in (w, s, b)]
+    rhs = torch.from_numpy(np.random.default_rng(K).integers(0, E, R).astype(np.int32)).cuda()
+    x = gpu.fill_normal_bf16(6100 + M, (R, M, K))
+    y = torch_bf16_bits(gpu.gather_qmm(x, w, s, b, rhs))
+    np.testing.assert_array_equal(y, torch_bf16_bits(gpu.gather_qmm(x, *more, rhs)))
