@@ -177,9 +177,9 @@ __device__ __forceinline__ uint16_t add_one(uint16_t a, uint16_t b) { return f2b
 
 // y = OP(a, b) elementwise: 8 values (16 bytes) per thread and array where
 // all three are 16-byte aligned and n is a multiple of 8, else one.
-// One value per thread was bound by issuing memory instructions: add of 10.5M
-// values 19.9 -> 10.7 us, silu_mul of 19.9M 33.3 -> 22.0 (now its expf and
-// division).  y may be a or b (each thread reads its values before it writes
+// One value per thread is bound by issuing memory instructions: add of 10.5M
+// values 19.9 -> 10.7 us, silu_mul of 19.9M 33.3 -> 22.0 (119 MB: the rate of
+// memory).  y may be a or b (each thread reads its values before it writes
 // them).
 template <uint16_t (*OP)(uint16_t, uint16_t), bool VEC>
 __global__ void __launch_bounds__(256) elementwise_kernel(const uint16_t* a, const uint16_t* b, uint16_t* y, int64_t n) {
@@ -199,13 +199,13 @@ __global__ void __launch_bounds__(256) elementwise_kernel(const uint16_t* a, con
   }
 }
 
+// (small arrays spread over more CUs one value per thread: 8 values a thread
+// from `from` values on)
 template <uint16_t (*OP)(uint16_t, uint16_t)>
-int launch_elementwise(const char* what, const uint16_t* a, const uint16_t* b, uint16_t* y, int64_t n,
+int launch_elementwise(const char* what, const uint16_t* a, const uint16_t* b, uint16_t* y, int64_t n, int64_t from,
                        hipStream_t stream) {
   if (n <= 0) return BMX_OK;
-  // (small arrays spread over more CUs one value per thread: 8 values a
-  // thread from 64 workgroups on)
-  const bool vec = n % 8 == 0 && n >= 64 * 2048 && aligned(a, 16) && aligned(b, 16) && aligned(y, 16);
+  const bool vec = n % 8 == 0 && n >= from && aligned(a, 16) && aligned(b, 16) && aligned(y, 16);
   const int64_t threads = vec ? n / 8 : n;
   const dim3 grid(static_cast<unsigned>((threads + 255) / 256));
   if (vec) hipLaunchKernelGGL((elementwise_kernel<OP, true>), grid, dim3(256), 0, stream, a, b, y, n);
@@ -243,11 +243,15 @@ int launch_argmax_partials(const uint2* part, int rows, int nblk, uint32_t* out,
 }
 
 int launch_silu_mul(const uint16_t* g, const uint16_t* u, uint16_t* y, int64_t n, hipStream_t stream) {
-  return launch_elementwise<silu_mul_one>("silu_mul", g, u, y, n, stream);
+  // one value per thread and 8, us: 359936 values 2.36 and 2.65, 749056 3.06
+  // and 3.36, 1048576 3.62 and 3.60, 2097152 5.23 and 4.82
+  return launch_elementwise<silu_mul_one>("silu_mul", g, u, y, n, 1 << 20, stream);
 }
 
 int launch_add(const uint16_t* a, const uint16_t* b, uint16_t* y, int64_t n, hipStream_t stream) {
-  return launch_elementwise<add_one>("add", a, b, y, n, stream);
+  // one value per thread and 8, us: 262144 values 2.16 and 2.25, 524288 2.43
+  // and 2.59, 749056 3.00 and 2.71, 2097152 4.84 and 3.59
+  return launch_elementwise<add_one>("add", a, b, y, n, 10 << 16, stream);
 }
 
 int launch_tokens_to_ids(const uint32_t* src, int32_t* dst, int n, hipStream_t stream) {

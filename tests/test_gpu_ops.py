@@ -319,10 +319,12 @@ def test_argmax_ties_nan_and_inf(gpu, orc, n):
     np.testing.assert_array_equal(gpu.argmax_rows(to_torch_bf16(x)).cpu().numpy(), want)
 
 
-@pytest.mark.parametrize("n", [131072, 131080, 131064, 131073])
+@pytest.mark.parametrize("n", [131072, 131080, 131064, 131073, 655352, 655360, 655361, 655368, 1048568, 1048576, 1048577,
+                               1048584])
 def test_elementwise_vector_path(gpu, n):
-    """Either side of the 8-values-per-thread rule, and operands 2 bytes off a
-    16-byte address: the same bits each way; add in place."""
+    """Either side of the 8-values-per-thread rules (add from 655360 values,
+    silu_mul from 1048576), and operands 2 bytes off a 16-byte address: the
+    same bits each way; add in place."""
     import torch
 
     a = gpu.fill_normal_bf16(18, (n + 1,), sigma=3.0)
