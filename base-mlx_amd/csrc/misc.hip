@@ -67,8 +67,12 @@ __device__ __forceinline__ void chain_publish(const DecodeChain& ch, uint32_t to
 // the largest value and the 16-byte unit it first stood in (three operations
 // per pair of values and three per unit, against five per value with an
 // index each), and looks the position up in that unit at the end.
-// 5 rows of 151936: 14.6 -> 8.2 us.
-__global__ void __launch_bounds__(kArgThreads)
+// 5 rows of 151936: 14.6 -> 8.2 us.  W: waves per SIMD that the registers
+// leave room for: 4 (one workgroup per CU, 10 loads) up to a row per CU, 8 (two,
+// 8 loads) for more rows, whose second workgroups else wait for the first (300
+// rows of 151937, not a multiple of 8: 57 us, 103 at 4).
+template <int B, int W>
+__global__ void __launch_bounds__(kArgThreads, W)
     argmax_kernel(const uint16_t* __restrict__ x, int64_t n, uint32_t* __restrict__ out, const DecodeChain ch) {
   const uint16_t* xr = x + static_cast<int64_t>(blockIdx.x) * n;
   float bv = -INFINITY;
@@ -76,14 +80,14 @@ __global__ void __launch_bounds__(kArgThreads)
   if (n % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
     const uint4* xv = reinterpret_cast<const uint4*>(xr);
     const int64_t nv = n / 8;
-    constexpr int B = 10;
     int64_t bj = -1;
     for (int64_t j0 = threadIdx.x; j0 < nv; j0 += static_cast<int64_t>(kArgThreads) * B) {
       uint4 d[B];
 #pragma unroll
       for (int u = 0; u < B; u++) d[u] = xv[min(j0 + static_cast<int64_t>(u) * kArgThreads, nv - 1)];
-      // (a unit past the end repeats the row's last one, which is never
-      // larger than itself seen before; a NaN loses every comparison)
+      // (a unit past the end repeats the row's last one: a thread that had not
+      // read that may take its value here, and means it -- see the min below;
+      // a NaN loses every comparison)
 #pragma unroll
       for (int u = 0; u < B; u++) {
         const uint32_t w[4] = {d[u].x, d[u].y, d[u].z, d[u].w};
@@ -228,7 +232,9 @@ int launch_argmax(const uint16_t* x, int64_t rows, int64_t n, uint32_t* out, hip
   if (rows > INT32_MAX) return set_error(BMX_E_SHAPE, "argmax: rows=%lld", (long long)rows);
   if (chain && (rows != 1 || !chain->io || !chain->ring)) return set_error(BMX_E_ARG, "argmax: chained hand-off of %lld rows", (long long)rows);
   const DecodeChain ch = chain ? *chain : DecodeChain{};
-  hipLaunchKernelGGL(argmax_kernel, dim3(static_cast<unsigned>(rows)), dim3(kArgThreads), 0, stream, x, n, out, ch);
+  const dim3 grid(static_cast<unsigned>(rows));
+  if (rows <= 256) hipLaunchKernelGGL((argmax_kernel<10, 4>), grid, dim3(kArgThreads), 0, stream, x, n, out, ch);
+  else hipLaunchKernelGGL((argmax_kernel<8, 8>), grid, dim3(kArgThreads), 0, stream, x, n, out, ch);
   return check_launch("argmax");
 }
 

@@ -319,6 +319,23 @@ def test_argmax_ties_nan_and_inf(gpu, orc, n):
     np.testing.assert_array_equal(gpu.argmax_rows(to_torch_bf16(x)).cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("n", [8, 8200, 8201, 81928])
+def test_argmax_more_rows_than_cus(gpu, n):
+    """Above 256 rows, other loads in flight per thread: ties, NaN and
+    infinities as one row at a time."""
+    x = np.repeat(torch_bf16_bits(gpu.fill_normal_bf16(22, (1, n))), 257, axis=0).copy()
+    x[1, n - 1] = x[1, n - 3] = 0x4200
+    x[2, :] = 0x7FC1
+    x[3, :n - 1] = 0x7FC1
+    x[3, n - 1] = 0xFF80
+    x[4, n // 2:] = 0x7F80
+    for r in range(5, 257):
+        x[r, (r * 7919) % n] = 0x4200
+    x = to_torch_bf16(x)
+    want = [int(gpu.argmax_rows(x[r:r + 1])[0]) for r in range(257)]
+    np.testing.assert_array_equal(gpu.argmax_rows(x).cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("n", [131072, 131080, 131064, 131073, 655352, 655360, 655361, 655368, 1048568, 1048576, 1048577,
                                1048584])
 def test_elementwise_vector_path(gpu, n):
