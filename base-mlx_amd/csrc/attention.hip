@@ -1339,7 +1339,11 @@ __global__ void __launch_bounds__(512) attn_flash32_kernel(const AttnParams p) {
     // ---- one of several splits of this tile: unnormalised partials ----
     if (t < p.M) {
       const int64_t row = (static_cast<int64_t>(blockIdx.z) * p.Hq + h) * p.M + t;
-      if (hf == 0) *reinterpret_cast<float2*>(p.part_ml + row * 2) = make_float2(m_run, l_run);
+      // a maximum of -inf tells the merge that the split has no weight for the
+      // row (no visible key; its O may hold 0 x NaN of hidden ones).  Scores
+      // that are all NaN leave it there too, with l NaN: any other maximum
+      // takes those into the row, which comes out NaN as it does unsplit
+      if (hf == 0) *reinterpret_cast<float2*>(p.part_ml + row * 2) = make_float2(l_run == l_run ? m_run : 0.0f, l_run);
       float* orow = p.part_o + row * kD + 4 * hf;
 #pragma unroll
       for (int dt = 0; dt < 4; dt++)
@@ -1396,10 +1400,7 @@ __global__ void __launch_bounds__(256) attn_flash_merge_kernel(const AttnParams 
     }
 #pragma unroll
     for (int u = 0; u < B; u++) {
-      // no key of the split visible to the row (its O may hold 0 x NaN of
-      // hidden keys).  Scores that are all NaN leave m at -inf too, with l NaN:
-      // those go on, so the row comes out NaN as it does unsplit
-      if (z0 + u >= ns || (ml[u].x == -INFINITY && ml[u].y == 0.0f)) continue;
+      if (z0 + u >= ns || ml[u].x == -INFINITY) continue;  // no weight in the split
       const float mn = fmaxf(m, ml[u].x);
       const float wa = __builtin_amdgcn_exp2f(m - mn), wb = __builtin_amdgcn_exp2f(ml[u].x - mn);
       l = l * wa + ml[u].y * wb;
