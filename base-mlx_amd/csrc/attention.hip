@@ -25,6 +25,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <functional>
 #include <mutex>
 
 #include "bmx_device.h"
@@ -1551,11 +1552,14 @@ int check_attention_shape(int Hq, int Hkv, int M, int D, int cap, int offset, co
 
 // Key blocks per split of a flash attention over `groups` head groups and
 // the key-block counts of its query tiles (a function of `tiles`, tq and the
-// mask): one workgroup per CU, so the time is about that of the longest
-// workgroup or of the mean load, in units of one key block (2.4 us measured),
-// with 2 blocks' worth per workgroup for its start and end and, once split,
-// 2 for the merge launch and the partials' traffic (Hq M 520 bytes per split,
-// written and read back at about 4 TB/s).  0: not split.
+// mask): one workgroup per CU, so the time is about the mean load or what the
+// longest workgroups that have to share a CU take, in units of one key block
+// (2.4 us measured), with 2 blocks' worth per workgroup for its start and end
+// and, once split, 2 for the merge launch and the partials' traffic (Hq M 520
+// bytes per split, written and read back at about 4 TB/s).  0: not split.
+// (By the longest workgroup alone, 64 q heads, 700 tokens over 8192, 176
+// workgroups, would split in two: 352 nearly equal ones, two rounds, 331 us
+// instead of 318.)
 int flash_split_blocks(int groups, int tiles, int tq, int Hq, int M, int offset, bool causal, size_t part_floats,
                        int64_t* splits_out) {
   constexpr int kCus = 256;
@@ -1565,24 +1569,37 @@ int flash_split_blocks(int groups, int tiles, int tq, int Hq, int M, int offset,
   };
   const int most = blocks(tiles - 1);
   *splits_out = 1;
-  if (tiles > 2 * kCus || most < 4) return 0;
+  // (no more than four workgroups per CU: the search stays a few thousand
+  // steps)
+  auto few = [&](int ns) { return static_cast<int64_t>(groups) * tiles * ns <= 4 * kCus; };
+  if (!few(2) || most < 4) return 0;
+  int part[2 * kCus];  // (tiles: at most that many)
   auto cost = [&](int bps) {
-    int64_t wgs = 0, sum = 0;
+    int64_t full = 0, sum = 0;
+    int parts = 0;
     for (int i = 0; i < tiles; i++) {
       const int n = blocks(i);
-      wgs += (n + bps - 1) / bps;
+      full += n / bps;
+      if (n % bps) part[parts++] = n % bps;
       sum += n;
     }
-    const double mean = static_cast<double>(groups) * (sum + 2 * wgs) / kCus;
+    const int64_t wgs = groups * (full + parts);
+    const double mean = static_cast<double>(groups) * (sum + 2 * (full + parts)) / kCus;
+    // of the 256 k + 1 longest workgroups, k + 1 share a CU
+    std::sort(part, part + parts, std::greater<int>());
+    double shared = 0.0;
+    for (int64_t k = 0; k * kCus < wgs; k++) {
+      const int64_t at = k * kCus;
+      const int n = at < groups * full ? bps : part[(at - groups * full) / groups];
+      shared = std::max(shared, (k + 1) * (n + 2.0));
+    }
     const double ns = (most + bps - 1) / bps;
     const double merge = ns > 1 ? 2.0 + ns * Hq * M * 1040.0 / 4.0e6 / 2.4 : 0.0;
-    return std::max(mean, bps + 2.0) * (groups * wgs > kCus ? 1.1 : 1.0) + merge;
+    return std::max(mean, shared) * (wgs > kCus ? 1.1 : 1.0) + merge;
   };
   int best = 0;
   double least = cost(most) * 0.9;  // a split has to promise 10%
-  // (no more than four workgroups per CU: the search stays a few thousand
-  // steps)
-  for (int ns = 2; ns <= 64 && (most + ns - 1) / ns >= 2 && static_cast<int64_t>(groups) * tiles * ns <= 4 * kCus; ns++) {
+  for (int ns = 2; ns <= 64 && (most + ns - 1) / ns >= 2 && few(ns); ns++) {
     const int bps = (most + ns - 1) / ns, n = (most + bps - 1) / bps;
     if (static_cast<size_t>(n) * Hq * M * (kD + 2) > part_floats) break;
     const double c = cost(bps);

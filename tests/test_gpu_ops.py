@@ -180,6 +180,18 @@ def test_attention_flash_key_split_nan_and_inf(gpu, Hq, Hkv, M, offset):
     assert ((one - two).abs()[fin] <= 2.0 ** -7 * one.abs()[fin] + 2e-3 * one[fin].abs().max()).all()
 
 
+def test_attention_flash_key_split_not_into_two_rounds(gpu):
+    """176 workgroups of about 134 key blocks: halved they are 352 nearly equal
+    ones for 256 CUs, no faster than whole, so the call has the unsplit bits."""
+    Hq, Hkv, M, offset = 64, 8, 700, 8192
+    q = gpu.fill_normal_bf16(67, (Hq, M, 128))
+    kc = gpu.fill_normal_bf16(68, (Hkv, offset + M, 128))
+    vc = gpu.fill_normal_bf16(69, (Hkv, offset + M, 128))
+    one = gpu.attention(q, kc, vc, offset, use_workspace=False)
+    two = gpu.attention(q, kc, vc, offset, workspace=gpu.attention_workspace(Hq, 16))
+    np.testing.assert_array_equal(torch_bf16_bits(one), torch_bf16_bits(two))
+
+
 def test_attention_workspace_reuse(gpu, orc):
     """One zero-filled workspace over calls of different split counts and row
     tilings: the arrival counters come back to zero after every call."""
