@@ -108,7 +108,8 @@ int launch_qmm_epi(QmmEpilogue epi, const uint16_t* x, const uint32_t* w, const 
                    const uint32_t* w2, const uint16_t* s2, const uint16_t* b2, const uint16_t* res, uint16_t* y, int M,
                    int N, int K, float* ws, size_t ws_floats, hipStream_t stream);
 // Whether launch_qmm_epi (one_launch: launch_qmm_segments, N the sum) takes
-// the few-rows kernel for the product, which reads MLX-layout weights.
+// the few-rows kernel for the product, which reads MLX-layout weights, rather
+// than the tile kernel on the group-major copy.
 bool qmm_few_rows(QmmEpilogue epi, int M, int N, int K, bool one_launch);
 // The same products over group-major copies of the weights (launch_qmm_repack):
 // W as [K/64][N][8] words and s|b as [K/64][N] words s | b << 16, so the

@@ -749,7 +749,12 @@ bool qmm_few_rows(QmmEpilogue epi, int M, int N, int K, bool one_launch) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64) return false;
   int splits, gps;
   qmm_split(M, N, K, &splits, &gps, epi == QMM_SWIGLU ? QBN / 2 : QBN);
-  return slab_plan(epi, M, N, K, one_launch ? 1 : splits).fits;
+  const SlabPlan s = slab_plan(epi, M, N, K, one_launch ? 1 : splits);
+  // against the group-major tile kernel: many row tiles of 128 columns gain
+  // nothing with a residual (a 4-layer 4B-shaped forward, o and down, of 1281
+  // and 1400 tokens: 1733 -> 1810 and 1803 -> 1883 us; 8B-shaped, 1024 tokens:
+  // equal); q|k|v and SwiGLU tiles do (8B-shaped, 640 tokens: 1840 -> 1617)
+  return s.fits && !(epi == QMM_RESIDUAL && s.bn == 128);
 }
 
 int launch_qmm_epi(QmmEpilogue epi, const uint16_t* x, const uint32_t* w, const uint16_t* s, const uint16_t* b,
