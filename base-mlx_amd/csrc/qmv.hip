@@ -1348,15 +1348,20 @@ int try_launch_qmvr(int S, const QmvParams& p, hipStream_t st) {
   const int C = p.K / 32, G = p.K / 64;
   if (!p.sb_vec || p.nseg != 1 || p.amax || C % S) return kNoFit;
   const int ni = C / S, slots = 64 / S;
-  // two rows of x are near the memory rate either way; from 4096 columns on
-  // the kernels below are ahead (151936 x 4096: 64.1 against 69.0 us)
-  if (MT == 2 && ni > 10) return kNoFit;
   constexpr int RPL = 2;
   const int RB = 8 * slots * RPL;
   if (RB * (G / 8) % 64 || RB * (G / 8) >= 1 << 20) return kNoFit;
   const size_t lds = static_cast<size_t>(MT) * C * (kChunkBytes + 4) + 16ull * MT + 8ull * RB * G;
   if (lds > 160 * 1024) return kNoFit;
   const int ntiles = (p.seg[0].rows + RB - 1) / RB;
+  // Few rows of x and long rows of W are near the memory rate either way, and
+  // the kernels below have the smaller tiles.  2 rows, from 3072 columns on:
+  // those (151936 x 4096: 64.1 against 69.0 us).  3 and 4 rows: at 3072
+  // columns those (151936: 74.5 against 76.6), from 4096 on those where the
+  // last round of tiles is empty by a tenth of all (100000 x 4096: 782 tiles,
+  // 69.6 against 77.6; 151936 x 4096: 1187 tiles, 100.2 against 96.3)
+  const int slack = ntiles % 256 ? 256 - ntiles % 256 : 0;
+  if (ni > 10 && (MT == 2 || (MT == 4 && (ni < 16 || 10 * slack > ntiles + slack)))) return kNoFit;
   auto go = [&](auto kern) {
     if (int rc = allow_lds(kern, lds)) return rc;
     hipLaunchKernelGGL(kern, dim3(std::min(256, ntiles)), dim3(kRThreads), lds, st, p, S, ntiles);
