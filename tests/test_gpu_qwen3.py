@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from _parity import Parity
-from _util import bf16_to_f32, l2_rel_err, torch_bf16_bits
+from _util import bf16_to_f32, l2_rel_err, to_torch_bf16, torch_bf16_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -288,9 +288,9 @@ def _write_projection(gpu, gm, layer, slot, arrays):
 
 
 def test_prefill_reads_weights_written_through_qlinear(gpu, orc):
-    """The prefill GEMMs read a group-major copy of each layer projection;
-    a projection written through the pointers of bmx_qwen3_qlinear is seen
-    by the next prefill: with layer 1's gate and down and layer 0's v
+    """A projection written through the pointers of bmx_qwen3_qlinear is seen
+    by the next prefill (here by the few-rows GEMMs, which read it in place;
+    the group-major copies are the next test's): with layer 1's gate and down and layer 0's v
     projection replaced in both models the logits follow the oracle's, and
     with the old weights written back they are the first prefill's bit for
     bit."""
@@ -313,6 +313,45 @@ def test_prefill_reads_weights_written_through_qlinear(gpu, orc):
         _write_projection(gpu, gm, *key, arrays)
     g2 = torch_bf16_bits(gm.forward(gm.new_cache(64), toks, all_logits=True))
     np.testing.assert_array_equal(g2, g0)
+
+
+# (shape, tokens of a forward whose q|k|v and gate|up GEMMs read the group-major
+# copies): K of 64 but not 128, where every forward's do, and down's too; SMALL
+# from about 1300 tokens on, while 40 take the few-rows GEMM, which does not
+# need the copies and leaves them as they are
+@pytest.mark.parametrize("shape,long", [(dict(hidden=576, inter=1472), 40), ({}, 1300)])
+def test_group_major_copies_follow_qlinear_writes(gpu, orc, shape, long):
+    """Weights written through bmx_qwen3_qlinear's pointers reach the
+    group-major copies before a forward reads those, also when a forward that
+    does not came between."""
+    gm, om = _pair(gpu, orc, seed=3, max_tokens=1300, **shape)
+    toks = {M: orc.fill_tokens(78, M, SMALL["vocab"]) for M in (9, 40, long)}
+
+    def forward(M):
+        return torch_bf16_bits(gm.forward(gm.new_cache(M), toks[M], all_logits=True))
+
+    def oracle(M):
+        return om.forward(om.new_cache(M), toks[M], all_logits=True)
+
+    first = {M: forward(M) for M in (long, 40, 9)}
+    old = {key: [a.copy() for a in gm.qlinear_numpy(*key)] for key in [(1, 4), (1, 6), (0, 2)]}
+    order = [40, long, 9] if long != 40 else [9, 40]
+    for (layer, slot), seed in [((1, 4), 5), ((1, 6), 7), ((0, 2), 6)]:
+        w, s, b = old[(layer, slot)]
+        new = (np.random.default_rng(seed).integers(0, 2**32, w.shape, dtype=np.uint32), s[::-1].copy(),
+               b[:, ::-1].copy())
+        _write_projection(gpu, gm, layer, slot, new)
+        for dst, src in zip(om.qlinear(layer, slot), new):
+            dst[...] = src
+    for M in order:
+        print(f"written weights, {M} tokens", flush=True)
+        got = forward(M)
+        assert not np.array_equal(got, first[M])
+        assert _check_logits(to_torch_bf16(got), oracle(M)) >= 0.9
+    for key, arrays in old.items():
+        _write_projection(gpu, gm, *key, arrays)
+    for M in order:
+        np.testing.assert_array_equal(forward(M), first[M])
 
 
 def test_qwen3_4b_shape_prefill_and_decode(gpu, orc):
