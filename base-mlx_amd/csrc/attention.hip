@@ -1624,8 +1624,8 @@ int launch_attention(const uint16_t* q, const uint16_t* k, const uint16_t* v, ui
                M > 1 ? 1 : 0, scale};
   const int rc = launch_decode(p, nullptr, ws, ws_floats, L_max, stream);
   if (rc != kNoFit) return rc;
-  // flash attention (no split workspace): a GQA group per workgroup when
-  // the heads per kv head are a power of two, else one head per workgroup
+  // flash attention: a GQA group per workgroup when the heads per kv head are
+  // a power of two, else one head per workgroup
   const int rep = Hq / Hkv;
   auto launch = [&](auto kern, int nw, int hg) {
     if (int e = allow_lds_ptr(reinterpret_cast<const void*>(kern), kFaLds)) return e;

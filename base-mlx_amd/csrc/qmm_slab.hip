@@ -138,7 +138,7 @@ __global__ void __launch_bounds__(64 * slab_waves(MT), slab_waves(MT) / 4) qmm_s
     }
   }
 
-  // ---- this lane's pieces of a slab: instruction i = wave + 8 k fills
+  // ---- this lane's pieces of a slab: instruction i = wave + NW k fills
   // pieces 64 i .. + 63 of the slot's x (W) part; the piece at position c of
   // row r is logical piece c ^ swizzle(r), so the operand reads below fall
   // in distinct banks ----
@@ -331,7 +331,10 @@ int launch_epi(const QmmParams& p, const SlabPlan& s, hipStream_t stream) {
 }  // namespace
 
 // The rule, from times of both kernels (us, tile kernel -> this one; weights
-// from memory):
+// from memory), where the LDS holds the whole split's s and b and two ring
+// slots (long K: else the tile kernel, as 5120 x 25600 at 33..48 and 97..384
+// rows, 83 and 87 us between 31.0 at 32 rows and 45.6 at 49; 4096 x 12288 at
+// 225..256 and from 289 on; 2560 x 9728 from 337):
 //   * up to 64 rows, any N: 9728 x 2560 20.7 -> 10.5 at 9 rows, 26.1 -> 16.4
 //     at 64; 151936 x 2560 141 -> 63 at 9, 133 -> 92 at 64;
 //   * more rows while the tiles are one round of the 256 CUs: 1024 x 2560
@@ -340,7 +343,8 @@ int launch_epi(const QmmParams& p, const SlabPlan& s, hipStream_t stream) {
 //     but 55.1 -> 73 at 2048 (512 tiles);
 //   * 64 columns per tile (half the x reuse, but twice the CUs) where those
 //     tiles fit the round, with K split to fill it: 2560 x 9728 at 37 rows
-//     29 -> 14.5 with 6 splits (unsplit 37); else 128 columns;
+//     29 -> 14.5 with 6 splits (unsplit 37), though 4096 x 12288 gains only
+//     47.7 -> 46.5 at 200 rows (28.8 at 128); else 128 columns;
 //   * not 128 columns in three or more row tiles that leave a fifth of the
 //     CUs idle: 8192 x 5120 at 300 rows (192 tiles) 60.5 -> 64.
 SlabPlan slab_plan(QmmEpilogue epi, int M, int N, int K, int max_splits) {
