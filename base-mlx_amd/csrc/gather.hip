@@ -506,8 +506,11 @@ int64_t gather_rows_further(int unit_rows, int M, int R) { return static_cast<in
 // 1536 x 2048, per route and by expert: 8 experts 16 routes 7.6 and 16.6, 80
 // routes 18.9 and 17.4; 32 experts 40 routes 16.7 and 18.3; 128 experts 160
 // routes 40.7 and 34.6, 1280 routes 259 and 58.  It picks the slower one by
-// more than 5% only near the line: at most 10% (1.4 us) over those shapes.
+// more than 5% only near the line, at most 12% over those shapes (4 experts of
+// 14336 x 4096, 6 routes: per route 33.1, by expert 29.5).
+// (Below 1.25 routes an expert the weights are hardly read twice.)
 bool gather_by_expert(int E, int M, int N, int K, int R) {
+  if (4ll * R < 5ll * E) return false;
   const double mb = static_cast<double>(N) * K * 0.5625e-6, used = mb * E * (1.0 - exp(-static_cast<double>(R) / E));
   const double per_route = 3.7 + M * (0.2 + 0.35 * K / 1024.0) + R * (0.005 + (1.0 + 0.4 * (M - 1)) * mb / 9.5) +
                            used / 16.0;
